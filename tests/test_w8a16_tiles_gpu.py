@@ -1,0 +1,91 @@
+"""The W8A16 block-tile kernel (w8a16_tile.h) on the GPU: every tile size the planner can pick, at
+shapes that leave a remainder in both directions of the tile, with fewer, as many and more K steps
+than the LDS ring has stages, and through each epilogue (plain, fp32 logits rows, gated MLP, RoPE
+with the cache write).
+
+The product is held to the W8A16 bars of test_kernels_gpu.py (relative Frobenius 1e-3; 1 fp16 ulp
+of the exact product plus fp32 accumulation noise, 1e-4 of the RMS); the fused epilogues equal the
+separate calls bit for bit, since both take the same K order."""
+
+from __future__ import annotations
+
+import numpy as np
+import pytest
+import torch
+
+from oracle import quant as OQ
+from turingserve_amd import hip_ops as K
+from turingserve_amd.qwen2 import rope_tables
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+# (M, N) -> tile on 256 CUs: each leaves partial tiles in M and N
+TILES = [(1000, 15988, "256x256"), (575, 17884, "256x192"), (1790, 2004, "128x128 two K groups"),
+         (1855, 1500, "128x96 four K groups"), (1000, 2004, "128x64 four K groups"),
+         (750, 2004, "64x96 four K groups"), (67, 17884, "128x96 two K groups"),
+         (131, 17884, "128x64 two K groups")]
+
+
+def _problem(M, N, Kd, fp16_scale=False):
+    g = torch.Generator().manual_seed(M * 7 + N + Kd)
+    wq = torch.randint(-127, 128, (N, Kd), generator=g, dtype=torch.int32).to(torch.int8)
+    scale = torch.rand(N, generator=g) * 0.01 + 0.001
+    scale = scale.half() if fp16_scale else scale
+    x = torch.randn(M, Kd, generator=g).half()
+    bias = (torch.randn(N, generator=g) * 0.5).half()
+    return x, wq, scale, bias
+
+
+@pytest.mark.parametrize("Kd", [128, 384, 640])
+@pytest.mark.parametrize("M,N,tile", TILES)
+def test_every_tile_against_the_oracle(M, N, tile, Kd):
+    x, wq, sc, bias = _problem(M, N, Kd, fp16_scale=Kd == 384)
+    y = K.w8a16_linear(x.cuda(), wq.cuda(), sc.cuda(), bias.cuda()).float().cpu().numpy()
+    ref = OQ.w8a16(x.numpy(), wq.numpy(), sc.numpy().astype(np.float64), bias.numpy(), np.float64)
+    assert np.linalg.norm(y - ref) / np.linalg.norm(ref) < 1e-3
+    rms = float(np.sqrt((ref ** 2).mean()))
+    ulp = np.spacing(np.abs(ref).astype(np.float16)).astype(np.float64)
+    assert (np.abs(y - ref.astype(np.float16).astype(np.float64)) <= ulp + 1e-4 * rms).all()
+
+
+@pytest.mark.parametrize("M,N,tile", TILES)
+def test_gated_epilogue_equals_the_pair(M, N, tile):
+    """The gated-MLP epilogue against the product then SiLU.up; also K of one 64-column step."""
+    inter = N // 16 * 8                                       # the separate kernel needs I % 8 == 0
+    for Kd in (64, 256):
+        x, wq, sc, bias = (t.cuda() for t in _problem(M, 2 * inter, Kd))
+        fused = K.w8a16_glu(x, wq, sc, bias)
+        assert torch.equal(fused, K.silu_mul(K.w8a16_linear(x, wq, sc, bias)))
+
+
+@pytest.mark.parametrize("M,N,tile", TILES)
+def test_logits_epilogue_equals_the_gathered_product(M, N, tile):
+    x, wq, sc, _ = (t.cuda() for t in _problem(M, N, 256))
+    rows = torch.randint(0, M, (M,), generator=torch.Generator().manual_seed(N)).cuda()
+    got = K.logits_int8(x, rows, wq, sc)
+    assert torch.equal(got, K.w8a16_linear(x[rows], wq, sc, None).float())
+
+
+@pytest.mark.parametrize("M,H,KVH", [(700, 12, 2), (1000, 12, 2), (1390, 12, 2), (1801, 12, 2),
+                                     (555, 100, 20), (1003, 84, 20)])
+def test_rope_epilogue_equals_the_separate_calls(M, H, KVH):
+    """Heads of 128 in tiles of 128 and 256 columns (700 rows: the plan's 64-column tile holds half
+    a head, so the fused call takes 128 columns), slots and positions out of range."""
+    from turingserve_amd.quant import LinearWeight
+
+    N, Kd, NB = (H + 2 * KVH) * 128, 256, 8 + M // 16
+    x, wq, sc, bias = (t.cuda() for t in _problem(M, N, Kd))
+    g = torch.Generator().manual_seed(M)
+    pos = torch.randint(-3, 600, (M,), generator=g).cuda()
+    slots = torch.randperm(NB * 16, generator=g)[:M].long()
+    slots[::5], slots[2] = -1, NB * 16 + 3
+    slots = slots.cuda()
+    cos, sin = rope_tables(128, 1e6, 512, DEV)
+    kv = torch.randn(2, NB, KVH, 16, 128, generator=g).half().cuda()
+    kv1, kv2 = kv.clone(), kv.clone()
+    qkv1 = K.linear_rope_kv_write(x, LinearWeight(wq, bias, sc), pos, cos, sin, H, KVH, 128,
+                                  kv1[0], kv1[1], slots)
+    qkv2 = K.w8a16_linear(x, wq, sc, bias)
+    assert K.rope_kv_write_(qkv2, pos, cos, sin, H, KVH, 128, kv2[0], kv2[1], slots)
+    assert torch.equal(qkv1, qkv2) and torch.equal(kv1, kv2)

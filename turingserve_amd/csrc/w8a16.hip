@@ -1196,6 +1196,12 @@ __global__ void __launch_bounds__(256) w8a16_wide_kernel(
   }
 }
 
+}  // namespace ts
+
+#include "w8a16_tile.h"
+
+namespace ts {
+
 // ------------------------------------------------------------------------------------------
 // Host side
 // ------------------------------------------------------------------------------------------
@@ -1228,6 +1234,7 @@ struct GemmPlan {
   int kw;          // skinny path: wavefronts per workgroup (the K split inside it)
   int gv;          // VALU path: threads per weight-row group (0: not this path)
   int gvr;         // VALU path: weight rows per thread
+  int tile;        // block-tile kernel (w8a16_tile.h) in place of the wide one; kTileNone: wide
 };
 
 // Variants a caller (a tuning table) may name instead of the planner's choice.
@@ -1331,6 +1338,57 @@ static int wide64_splits(int M, int N, int K, int cus) {
   return splits;
 }
 
+// Block tiles (w8a16_tile_kernel) that replace a wide plan with one K split past M = 64; `rows` x
+// `cols` of Y^T, K steps of `bk`. The four with bk = 128 and four K groups sum K in the same order.
+enum GemmTile : int {
+  kTileNone = 0, kTile256x256, kTile256x192, kTile128x128k2, kTile128x96k4, kTile128x64k4,
+  kTile64x96k4, kTile128x96k2, kTile128x64k2
+};
+struct TileSize { int rows, cols, bk; };
+constexpr TileSize kTileSizes[] = {{0, 0, 0},     {256, 256, 64}, {256, 192, 64},
+                                   {128, 128, 128}, {128, 96, 128}, {128, 64, 128},
+                                   {64, 96, 128}, {128, 96, 64},  {128, 64, 64}};
+static int64_t tile_count(int t, int M, int N) {
+  const TileSize& s = kTileSizes[t];
+  return (int64_t)((N + s.rows - 1) / s.rows) * ((M + s.cols - 1) / s.cols);
+}
+
+// Which block tile, for a product whose wide plan does not split K (measured with cold weights,
+// wide plan -> block tile; one workgroup per CU unless said otherwise):
+//  * 256 x 256 or 256 x 192 where the output fills its resident rounds well enough that the
+//    larger operand blocks pay: at least 9/10 (16384 x 8192 at M = 2048: 620 -> 482 us) and 25/32
+//    of rounds x CUs x tile (17920 x 1536: M = 560 44.8 -> 41.3 us, M = 1856 138 -> 121 us; at
+//    M = 1024 and 1400, 0.73 and 0.67 of the rounds, they measured 4 and 8 % slower);
+//  * the smallest of 64 x 96, 128 x 64, 128 x 96 (four K groups) and 128 x 128 (two) that fits one
+//    round of one workgroup per CU, so that the most CUs share the work, while it covers 0.7
+//    of them (2048 x 1536: M = 560 / 768 / 1400 / 1856 11.5 / 11.9 / 17.8 / 20.7 -> 10.3 / 10.6 /
+//    16.0 / 18.5 us; 1536 x 1536 at M = 1856 20.0 -> 16.2; 1536 x 8960: M = 1400 / 1856 71.1 / 85.8 ->
+//    55.9 / 60.0; below the 0.7, 128 x 32 wide tiles stay: 1536 x 1536 at M = 560 8.9 against 9.9);
+//  * 128 x 96 or 128 x 64 with two K groups and two workgroups per CU, whichever pads fewer rows,
+//    for a wide product of few rows (17920 x 1536: M = 72 / 130 / 192 / 256 20.8 / 23.7 / 25.1 /
+//    31.0 -> 17.4 / 22.2 / 24.1 / 29.2 us).
+static int pick_tile(int M, int N, int K, int cus) {
+  if (K % kTileBK != 0) return kTileNone;
+  auto fills = [&](int t, int num, int den) {
+    const int64_t rounds = (tile_count(t, M, N) + cus - 1) / cus;
+    return (int64_t)M * N * den >=
+           num * rounds * cus * ((int64_t)kTileSizes[t].rows * kTileSizes[t].cols);
+  };
+  if (fills(kTile256x256, 9, 10)) return kTile256x256;
+  if (fills(kTile256x192, 25, 32)) return kTile256x192;
+  if (K % 128 == 0 && tile_count(kTile128x128k2, M, N) <= cus) {
+    for (int t : {kTile64x96k4, kTile128x64k4, kTile128x96k4, kTile128x128k2})
+      if (tile_count(t, M, N) <= cus) return tile_count(t, M, N) * 10 >= 7LL * cus ? t : kTileNone;
+  }
+  if (M <= 256 && tile_count(kTile128x96k2, M, N) * 2 > cus) {
+    const int r64 = (M + 63) / 64 * 64, r96 = (M + 95) / 96 * 96;
+    const int t = r64 <= r96 && tile_count(kTile128x64k2, M, N) <= 2LL * cus ? kTile128x64k2
+                                                                            : kTile128x96k2;
+    if (tile_count(t, M, N) <= 2LL * cus) return t;
+  }
+  return kTileNone;
+}
+
 // The plan of a variant with `splits` K splits (0: the variant's own rule). kVarAuto: weight
 // streaming when use_small_path says so; else 128 x 128 tiles (two workgroups per CU; the most
 // work per CU of the shapes measured) once they cover more than half the CUs and M is past 64
@@ -1346,6 +1404,7 @@ static int wide64_splits(int M, int N, int K, int cus) {
 // and GLU mode plans them as 128 x 64.
 static GemmPlan plan_gemm_v(int M, int N, int K, int cus, int variant, int splits,
                             bool glu = false) {
+  const bool own_rule = variant == kVarAuto;
   if (variant == kVarGemv || (variant == kVarAuto && use_gemv(M, N, K))) {
     GemmPlan p{false, 1, 0, 0, 1, K, 0, 0, 0, 0};
     gemv_shape(M, K, glu, &p);
@@ -1438,6 +1497,7 @@ static GemmPlan plan_gemm_v(int M, int N, int K, int cus, int variant, int split
     p.k_per_split = steps * kTileBK;
     p.splits = (K + p.k_per_split - 1) / p.k_per_split;
   }
+  if (own_rule && M > 64 && p.splits == 1) p.tile = pick_tile(M, N, K, cus);
   return p;
 }
 
@@ -1584,9 +1644,38 @@ static int w8a16_launch(const half_t* xp, int64_t ldx, const int8_t* wq, const v
     if (part) reduce(part);
   } else {
     float* part = p.splits > 1 ? static_cast<float*>(workspace) : nullptr;
+    const bool fast = K % kTileBK == 0 && aligned(wq, 16);   // weight DMA, no K tail
+    if (p.tile != kTileNone && fast) {
+      int t = p.tile;
+      // RoPE needs whole heads of 128 columns per tile (same K order, see GemmTile)
+      if (io.rope_cos && t == kTile64x96k4) t = kTile128x64k4;
+      const TileSize& ts = kTileSizes[t];
+      const dim3 grid(glu ? (io.glu + ts.rows / 2 - 1) / (ts.rows / 2) : (N + ts.rows - 1) / ts.rows,
+                      (M + ts.cols - 1) / ts.cols);
+#define TS_TILE_CASE(ID, ...)                                                                      \
+  case ID: {                                                                                       \
+    using Shape = TileShape<__VA_ARGS__>;                                                          \
+    static_assert(Shape::kTN == kTileSizes[ID].rows && Shape::kTM == kTileSizes[ID].cols &&        \
+                  Shape::kBK == kTileSizes[ID].bk, "the planner's table");                         \
+    w8a16_tile_kernel<__VA_ARGS__><<<grid, Shape::kThreads, 0, s>>>(                               \
+        xp, ldx, wq, scale, scale_is_fp16, bp, yp, ldy, M, N, K, io);                              \
+    break;                                                                                         \
+  }
+      switch (t) {
+        TS_TILE_CASE(kTile256x256, 2, 4, 4, 2, 1, 1, 3)
+        TS_TILE_CASE(kTile256x192, 2, 3, 4, 2, 1, 1, 3)
+        TS_TILE_CASE(kTile128x128k2, 2, 2, 2, 2, 2, 2, 3)
+        TS_TILE_CASE(kTile128x96k4, 2, 3, 2, 1, 4, 2, 3)
+        TS_TILE_CASE(kTile128x64k4, 2, 2, 2, 1, 4, 2, 4)
+        TS_TILE_CASE(kTile64x96k4, 1, 3, 2, 1, 4, 2, 4)
+        TS_TILE_CASE(kTile128x96k2, 2, 3, 2, 1, 2, 1, 3)
+        TS_TILE_CASE(kTile128x64k2, 2, 2, 2, 1, 2, 1, 3)
+      }
+#undef TS_TILE_CASE
+      return TS_OK;
+    }
     const int tiles_n = glu ? (io.glu + p.bn / 2 - 1) / (p.bn / 2) : (N + p.bn - 1) / p.bn;
     const dim3 grid(tiles_n, (M + p.bm - 1) / p.bm, p.splits);
-    const bool fast = K % kTileBK == 0 && aligned(wq, 16);   // weight DMA, no K tail
 #define TS_WIDE_LAUNCH(WNV, WMV)                                                                   \
   if (fast)                                                                                        \
     w8a16_wide_kernel<WNV, WMV, wide_prefetch(true, WMV), true, false><<<grid, 256, 0, s>>>(       \
