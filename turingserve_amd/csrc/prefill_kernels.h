@@ -212,9 +212,13 @@ __global__ void __launch_bounds__(NW * 64) prefill_stream_kernel(
 
 
 // ------------------------------------------------------------------------------------------
-// LDS-tiled prefill (D = 128, the Qwen2.5 attention shapes).
+// LDS-tiled prefill (D = 128 and 64, the Qwen2.5 attention shapes).
 //
-// Workgroup = 128 query rows of one query head, four wavefronts of 32 rows each. Every 64-key
+// Workgroup = 128 query rows of one query head, four wavefronts of 32 rows each; with two key
+// groups (D = 64) 64 rows, two wavefronts per group, the groups taking the steps in turn and meeting
+// in LDS at the end: a workgroup alone on its CU is bound by the chain of one step (reads, MFMAs,
+// softmax, ~1.2 us at D = 64), which two groups halve (five ragged chunks, 2060 rows on 14 heads:
+// 31.8 -> 23.8 us; the 32-row stream kernel 35.7). Every 64-key
 // step (four 16-token blocks) is staged once in LDS and shared by the four wavefronts: K in its
 // natural [key][dim] layout, V transposed to [dim][key] (16 bytes of padding per row keep the
 // 16-lane groups of each 16-byte read on distinct banks). Wavefront w stages block w of the
@@ -243,6 +247,11 @@ constexpr int kTileRows = 128;
 constexpr int kTileKeys = 64;
 constexpr int kTileThreads = 256;
 constexpr int kPrefillMinSteps = 4;   // fewest 64-key steps a split is given
+// Query rows of a tile whose four wavefronts form `ks` key groups.
+constexpr int tile_rows(int ks) { return kTileRows / ks; }
+// Workgroups per CU that the registers and the LDS leave room for.
+template <int D, int KS>
+constexpr int kTilePerCu = D == 64 && KS == 1 ? 3 : 2;
 constexpr int kMergeRows = 2;         // rows per merge thread (8 dims each)
 
 template <int D>
@@ -335,13 +344,24 @@ __device__ __forceinline__ int first_cut_tile(int q_len, int prefix, int seq_len
   return -1;
 }
 
+// What a launch does where a host bound is below the batch's real lengths: it computes rows
+// [0, rows) of a sequence, and one longer than `seq` runs its tiles unsplit (the plan's slots hold
+// the splits of shorter ones). Without caps the launch's lowest tiles become NaN rows.
+struct PrefillCaps {
+  int rows, seq;
+};
+constexpr PrefillCaps kNoCaps{1 << 30, 1 << 30};
+constexpr int kUnsplit = 1 << 30;
+
+// q_len: the rows the launch computes, q_all: the sequence's rows.
 struct PrefillSeq {
-  int q_start, q_len, seq_len, prefix;
+  int q_start, q_len, q_all, seq_len, prefix;
 };
 
 __device__ __forceinline__ PrefillSeq prefill_seq(const int* __restrict__ qsl,
                                                   const int* __restrict__ seq_lens, int b,
-                                                  int64_t num_tokens, int max_blocks) {
+                                                  int64_t num_tokens, int max_blocks,
+                                                  int row_cap = kNoCaps.rows) {
   PrefillSeq p;
   p.q_start = __builtin_amdgcn_readfirstlane(qsl[b]);
   p.q_len = __builtin_amdgcn_readfirstlane(qsl[b + 1]) - p.q_start;
@@ -349,22 +369,26 @@ __device__ __forceinline__ PrefillSeq prefill_seq(const int* __restrict__ qsl,
   int sl = __builtin_amdgcn_readfirstlane(seq_lens[b]);
   p.seq_len = sl < 0 ? 0 : (sl > max_blocks * kBlockSize ? max_blocks * kBlockSize : sl);
   p.prefix = p.seq_len - p.q_len;
+  p.q_all = p.q_len;
+  p.q_len = p.q_len < row_cap ? p.q_len : row_cap;
   return p;
 }
 
 // Workspace of the split path: per-split rows O (unnormalised) [slots_total][128][D] fp32, then
 // (m, l) pairs [slots_total][128][2] fp32, slots_total = P * H * slots.
-template <int D>
+template <int D, int KS>
 __device__ __forceinline__ void prefill_tile_body(
     const half_t* __restrict__ q, int64_t q_st, int64_t q_sh, half_t* __restrict__ out,
     int64_t o_st, int64_t num_tokens, const half_t* __restrict__ kc,
     const half_t* __restrict__ vc, int64_t NB, const int* __restrict__ bt, int64_t bt_st,
     int max_blocks, const int* __restrict__ seq_lens, const int* __restrict__ qsl,
-    int num_decode, int H, int KVH, float sl2, int smax, int slots, int P,
+    int num_decode, int H, int KVH, float sl2, int smax, int slots, int P, PrefillCaps caps,
     float* __restrict__ ws,
     int bx, char* __restrict__ lds) {
-  static_assert(D == 128, "the staging roles below assume D = 128");
+  static_assert(D == 128 || D == 64, "the staging roles below");
+  static_assert(KS == 1 || KS == 2, "one or two key groups");
   using L = TileLayout<D>;
+  constexpr int RW = 4 / KS, TR = tile_rows(KS);   // row wavefronts per key group, tile rows
   constexpr int KK = D / 16;                       // k-steps of S^T
   constexpr int DT = D / 32;                       // 32-dim tiles of O^T
 
@@ -393,25 +417,28 @@ __device__ __forceinline__ void prefill_tile_body(
   const int b = num_decode + pi;
   const int tid = threadIdx.x, lane = tid & 63;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int kg = w / RW, rw = w % RW;              // key group, row wavefront
   const int r = lane & 31, hh = lane >> 5;
 
-  const PrefillSeq sq = prefill_seq(qsl, seq_lens, b, num_tokens, max_blocks);
+  const PrefillSeq sq = prefill_seq(qsl, seq_lens, b, num_tokens, max_blocks, caps.rows);
+  if (sq.seq_len > caps.seq) smax = kUnsplit;
   if (slot == slots - 1) {
     // Rows of tiles the launch misses are written by no other workgroup.
-    const int cut = first_cut_tile(sq.q_len, sq.prefix, sq.seq_len, smax, kTileRows, slots);
+    const int cut = first_cut_tile(sq.q_len, sq.prefix, sq.seq_len, smax, TR, slots);
     if (cut >= 0) {
-      const int m_end = (cut + 1) * kTileRows < sq.q_len ? (cut + 1) * kTileRows : sq.q_len;
+      const int m_end = (cut + 1) * TR < sq.q_len ? (cut + 1) * TR : sq.q_len;
       poison_rows<D>(out, o_st, sq.q_start, 0, m_end, h);
     }
+    if (sq.q_all > sq.q_len) poison_rows<D>(out, o_st, sq.q_start, sq.q_len, sq.q_all, h);
   }
-  const TileSlot tsl = tile_slot(slot, sq.q_len, sq.prefix, sq.seq_len, smax, kTileRows);
+  const TileSlot tsl = tile_slot(slot, sq.q_len, sq.prefix, sq.seq_len, smax, TR);
   if (tsl.tile < 0) return;
-  const int m0 = tsl.tile * kTileRows;
-  const int last = (m0 + kTileRows < sq.q_len ? m0 + kTileRows : sq.q_len) - 1;
+  const int m0 = tsl.tile * TR;
+  const int last = (m0 + TR < sq.q_len ? m0 + TR : sq.q_len) - 1;
   int kv_hi = sq.prefix + last + 1 < sq.seq_len ? sq.prefix + last + 1 : sq.seq_len;
   kv_hi = kv_hi < 0 ? 0 : kv_hi;
   const int nblk = (kv_hi + kBlockSize - 1) / kBlockSize;
-  const int r0 = m0 + 32 * w;                      // first query row of this wavefront
+  const int r0 = m0 + 32 * rw;                     // first query row of this wavefront
   const int row = r0 + r;
   const bool row_ok = row < sq.q_len;
 
@@ -427,39 +454,45 @@ __device__ __forceinline__ void prefill_tile_body(
   const int64_t head_off = (int64_t)kvh * kBlockSize * D;
   const int64_t blk_stride = (int64_t)KVH * kBlockSize * D;
   const int* btrow = bt + (int64_t)b * bt_st;
-  // Staging: wavefront w loads block w of the step. K: lane -> token lane / 4, dims
-  // 32 (lane % 4) .. +31 (four 16-byte pieces). V: lane -> tokens {4 v + i, 8 + 4 v + i}
-  // (v = lane / 32, i = 0..3), dims 4 (lane % 32) .. +3 (eight 8-byte pieces; 32 lanes cover a
-  // token row): exactly the eight keys of V^T piece 2w + v, so each lane writes four whole
+  // Staging: wavefront rw of a key group loads blocks rw, rw + RW, .. of the group's step. K: lane -> token lane / 4, dims
+  // (D / 4) (lane % 4) .. + D / 4 - 1 (16-byte pieces). V: lane -> tokens {4 v + i, 8 + 4 v + i}
+  // (v = lane / 32, i = 0..3), dims VD (lane % 32) .. + VD - 1 (eight pieces of VD dims; 32 lanes
+  // cover a token row): exactly the eight keys of V^T piece 2 block + v, so each lane writes VD whole
   // 16-byte pieces, one per dim.
-  half8_t skA[4], skB[4];                         // two steps in flight (register double buffer)
-  half4_t svA[8], svB[8];
-  auto stage_load = [&](int st, half8_t (&sk)[4], half4_t (&sv)[8]) {
-    int bi = st * 4 + w;
+  constexpr int KP = D / 32, VD = D / 32;
+  typedef typename HalfVec<VD>::type VPart;
+  half8_t skA[KS][KP], skB[KS][KP];               // two steps in flight (register double buffer)
+  VPart svA[KS][8], svB[KS][8];
+  auto load_block = [&](int bi, half8_t (&sk)[KP], VPart (&sv)[8]) {
     bi = bi < nblk ? bi : nblk - 1;                // past the tile's keys: repeat (masked)
     const int64_t off = clamp_block(btrow[bi], NB) * blk_stride + head_off;
-    const half_t* kp = kc + off + (lane >> 2) * D + 32 * (lane & 3);
+    const half_t* kp = kc + off + (lane >> 2) * D + 8 * KP * (lane & 3);
 #pragma unroll
-    for (int i = 0; i < 4; ++i) sk[i] = ld<half8_t>(kp + 8 * i);
-    const half_t* vp = vc + off + 4 * (lane >> 5) * D + 4 * (lane & 31);
+    for (int i = 0; i < KP; ++i) sk[i] = ld<half8_t>(kp + 8 * i);
+    const half_t* vp = vc + off + 4 * (lane >> 5) * D + VD * (lane & 31);
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      sv[i] = ld<half4_t>(vp + i * D);
-      sv[4 + i] = ld<half4_t>(vp + (8 + i) * D);
+      sv[i] = ld<VPart>(vp + i * D);
+      sv[4 + i] = ld<VPart>(vp + (8 + i) * D);
     }
   };
-  auto stage_store = [&](int st, int buf, const half8_t (&sk)[4], const half4_t (&sv)[8]) {
-    char* kb = lds + buf * L::STAGE;
-    char* vb = kb + L::KBYTES;
-    char* kd = kb + (16 * w + (lane >> 2)) * L::KROW + 64 * (lane & 3);
+  auto stage_load = [&](int st, half8_t (&sk)[KS][KP], VPart (&sv)[KS][8]) {
 #pragma unroll
-    for (int i = 0; i < 4; ++i) ts::st<half8_t>(kd + 16 * i, sk[i]);
+    for (int u = 0; u < KS; ++u) load_block(st * 4 + rw + RW * u, sk[u], sv[u]);
+  };
+  char* glds = lds + kg * 2 * L::STAGE;            // this key group's two buffers
+  auto store_block = [&](int st, int blk, int buf, const half8_t (&sk)[KP], const VPart (&sv)[8]) {
+    char* kb = glds + buf * L::STAGE;
+    char* vb = kb + L::KBYTES;
+    char* kd = kb + (16 * blk + (lane >> 2)) * L::KROW + 16 * KP * (lane & 3);
+#pragma unroll
+    for (int i = 0; i < KP; ++i) ts::st<half8_t>(kd + 16 * i, sk[i]);
     // V^T: the eight keys of this lane, transposed; keys at or past kv_hi are zeroed (a reused
     // block may hold NaN there, and 0 * NaN would reach the output).
     const int vv = lane >> 5;
-    const int key0 = st * kTileKeys + 16 * w + 4 * vv;
-    const half4_t z4 = {0, 0, 0, 0};
-    half4_t x[8];
+    const int key0 = st * kTileKeys + 16 * blk + 4 * vv;
+    const VPart z4 = (VPart)((half_t)0);
+    VPart x[8];
 #pragma unroll
     for (int i = 0; i < 8; ++i) x[i] = sv[i];
     if ((st + 1) * kTileKeys > kv_hi) {            // the tile's last step only
@@ -469,13 +502,17 @@ __device__ __forceinline__ void prefill_tile_body(
         x[4 + i] = key0 + 8 + i < kv_hi ? sv[4 + i] : z4;
       }
     }
-    const int piece = 2 * w + vv;
+    const int piece = 2 * blk + vv;
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int d = 4 * (lane & 31) + j;
+    for (int j = 0; j < VD; ++j) {
+      const int d = VD * (lane & 31) + j;
       const half8_t t8 = {x[0][j], x[1][j], x[2][j], x[3][j], x[4][j], x[5][j], x[6][j], x[7][j]};
       ts::st<half8_t>(vb + d * L::VROW + 16 * (piece ^ vt_swz(d)), t8);
     }
+  };
+  auto stage_store = [&](int st, int buf, const half8_t (&sk)[KS][KP], const VPart (&sv)[KS][8]) {
+#pragma unroll
+    for (int u = 0; u < KS; ++u) store_block(st, rw + RW * u, buf, sk[u], sv[u]);
   };
 
   float16_t o[DT];
@@ -489,7 +526,7 @@ __device__ __forceinline__ void prefill_tile_body(
   auto compute = [&](int st, int buf) {
     const int k0 = st * kTileKeys;
     if (r0 >= sq.q_len || k0 > sq.prefix + r0 + 31) return;   // nothing visible to this wave
-    const char* kb = lds + buf * L::STAGE;
+    const char* kb = glds + buf * L::STAGE;
     const char* vb = kb + L::KBYTES;
     // S^T for both key halves: the two MFMA chains alternate and the K operands of k-step
     // kk + 1 are requested before the MFMAs of k-step kk, so each LDS read has two MFMAs of
@@ -557,29 +594,62 @@ __device__ __forceinline__ void prefill_tile_body(
             p[u], o[t]);
   };
 
-  // Step s sits in LDS buffer (s - lo) % 2 while the registers hold step s + 1 (loaded one
-  // step earlier) and receive step s + 2. The loads are unconditional (past the range they
-  // repeat its last step, a cache hit), so each wait covers exactly the registers it needs.
+  // The key groups take the steps in turn: iteration i of group kg is step lo + KS i + kg. It sits
+  // in LDS buffer i % 2 while the registers hold iteration i + 1 (loaded one iteration earlier)
+  // and receive iteration i + 2. The loads are unconditional (past the range they repeat its last
+  // step, a cache hit), so each wait covers exactly the registers it needs.
   if (tsl.lo < tsl.hi) {
     const int hi1 = tsl.hi - 1;
-    stage_load(tsl.lo, skA, svA);
-    stage_load(tsl.lo + 1 < hi1 ? tsl.lo + 1 : hi1, skB, svB);
-    stage_store(tsl.lo, 0, skA, svA);
+    const int nit = (tsl.hi - tsl.lo + KS - 1) / KS;
+    auto step = [&](int i) { return tsl.lo + KS * i + kg; };
+    auto in_range = [&](int i) { return step(i) < hi1 ? step(i) : hi1; };
+    auto run = [&](int i, int buf) {
+      if (KS == 1 || step(i) < tsl.hi) compute(step(i), buf);
+    };
+    stage_load(in_range(0), skA, svA);
+    stage_load(in_range(1), skB, svB);
+    stage_store(in_range(0), 0, skA, svA);
     __syncthreads();
-    for (int st = tsl.lo; st < tsl.hi; st += 2) {
-      stage_load(st + 2 < hi1 ? st + 2 : hi1, skA, svA);
-      compute(st, 0);
-      if (st + 1 < tsl.hi) stage_store(st + 1, 1, skB, svB);
+    for (int i = 0; i < nit; i += 2) {
+      stage_load(in_range(i + 2), skA, svA);
+      run(i, 0);
+      if (i + 1 < nit) stage_store(in_range(i + 1), 1, skB, svB);
       __syncthreads();
-      if (st + 1 >= tsl.hi) break;
-      stage_load(st + 3 < hi1 ? st + 3 : hi1, skB, svB);
-      compute(st + 1, 1);
-      if (st + 2 < tsl.hi) stage_store(st + 2, 0, skA, svA);
+      if (i + 1 >= nit) break;
+      stage_load(in_range(i + 3), skB, svB);
+      run(i + 1, 1);
+      if (i + 2 < nit) stage_store(in_range(i + 2), 0, skA, svA);
       __syncthreads();
     }
   }
 
-  const float lt = pair_sum(l);
+  float lt = pair_sum(l);
+  if constexpr (KS == 2) {
+    // The second key group hands its state of each row over in LDS (the stages are free); the
+    // first one merges it into its own (a group without a visible key has m = -inf, weight 0).
+    float* sx = reinterpret_cast<float*>(lds) + rw * (16 * DT + 2) * 64 + lane;
+    static_assert(RW * (16 * DT + 2) * 64 * sizeof(float) <= 4 * L::STAGE, "the hand-over fits");
+    if (kg == 1) {
+#pragma unroll
+      for (int t = 0; t < DT; ++t)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) sx[(16 * t + e) * 64] = o[t][e];
+      sx[16 * DT * 64] = m;
+      sx[(16 * DT + 1) * 64] = lt;
+    }
+    __syncthreads();
+    if (kg == 1) return;
+    const float m1 = sx[16 * DT * 64], l1 = sx[(16 * DT + 1) * 64];
+    const float mm = fmaxf(m, m1);
+    const float w0 = m == -INFINITY ? 0.f : fast_exp2(m - mm);
+    const float w1 = m1 == -INFINITY ? 0.f : fast_exp2(m1 - mm);
+    lt = lt * w0 + l1 * w1;
+    m = mm;
+#pragma unroll
+    for (int t = 0; t < DT; ++t)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) o[t][e] = o[t][e] * w0 + sx[(16 * t + e) * 64] * w1;
+  }
   if (!row_ok) return;
   if (tsl.nsplit == 1) {
     const float inv = lt == 0.f ? 0.f : 1.f / lt;
@@ -597,7 +667,7 @@ __device__ __forceinline__ void prefill_tile_body(
     // split's state (ops/triton_decode_attention.py:190-192).
     const int64_t wslot = ((int64_t)pi * H + h) * slots + slot;
     const int64_t total = (int64_t)P * H * slots;
-    float* wo = ws + (wslot * kTileRows + 32 * w + r) * D + 4 * hh;
+    float* wo = ws + (wslot * TR + 32 * rw + r) * D + 4 * hh;
 #pragma unroll
     for (int t = 0; t < DT; ++t)
 #pragma unroll
@@ -605,24 +675,24 @@ __device__ __forceinline__ void prefill_tile_body(
         ts::st<float4_t>(wo + 32 * t + 8 * j,
                          float4_t{o[t][4 * j], o[t][4 * j + 1], o[t][4 * j + 2], o[t][4 * j + 3]});
     if (hh == 0) {
-      float* wml = ws + total * kTileRows * D + (wslot * kTileRows + 32 * w + r) * 2;
+      float* wml = ws + total * TR * D + (wslot * TR + 32 * rw + r) * 2;
       wml[0] = m;
       wml[1] = lt;
     }
   }
 }
 
-template <int D>
-__global__ void __launch_bounds__(kTileThreads, 2) prefill_tile_kernel(
+template <int D, int KS>
+__global__ void __launch_bounds__(kTileThreads, (kTilePerCu<D, KS>)) prefill_tile_kernel(
     const half_t* __restrict__ q, int64_t q_st, int64_t q_sh, half_t* __restrict__ out,
     int64_t o_st, int64_t num_tokens, const half_t* __restrict__ kc,
     const half_t* __restrict__ vc, int64_t NB, const int* __restrict__ bt, int64_t bt_st,
     int max_blocks, const int* __restrict__ seq_lens, const int* __restrict__ qsl,
-    int num_decode, int H, int KVH, float sl2, int smax, int slots, int P,
+    int num_decode, int H, int KVH, float sl2, int smax, int slots, int P, PrefillCaps caps,
     float* __restrict__ ws) {
-  __shared__ __attribute__((aligned(16))) char lds[2 * TileLayout<D>::STAGE];
-  prefill_tile_body<D>(q, q_st, q_sh, out, o_st, num_tokens, kc, vc, NB, bt, bt_st, max_blocks,
-                       seq_lens, qsl, num_decode, H, KVH, sl2, smax, slots, P, ws,
+  __shared__ __attribute__((aligned(16))) char lds[2 * KS * TileLayout<D>::STAGE];
+  prefill_tile_body<D, KS>(q, q_st, q_sh, out, o_st, num_tokens, kc, vc, NB, bt, bt_st, max_blocks,
+                       seq_lens, qsl, num_decode, H, KVH, sl2, smax, slots, P, caps, ws,
                        (int)blockIdx.x, lds);
 }
 
@@ -633,15 +703,19 @@ __global__ void __launch_bounds__(kTileThreads, 2) prefill_tile_kernel(
 // slot_rows rows, the thread's rows at row0 + kMergeRowStride * k of each slot, and go to dst[k]
 // (nullptr: not wanted). The partials are taken kMergeBatch at a time, all of a batch's loads
 // requested together (cnt is uniform over the workgroup, so the unused ones are not issued).
-constexpr int kMergeRowStride = kTileThreads / 16;   // 16 rows per pass of a 256-thread group
+template <int D>
+constexpr int kMergeRowStride = kTileThreads / (D / 8);   // rows per pass of a 256-thread group
 constexpr int kMergeBatch = 4;
+// Workgroups per tile of the split tiles' merge.
+template <int D, int KS>
+constexpr int kMergeParts = tile_rows(KS) / (kMergeRowStride<D> * kMergeRows);
 
 template <int D>
 __device__ __forceinline__ void merge_partials(const float* __restrict__ ws, int64_t total_slots,
                                                int slot_rows, int64_t base, int cnt, int row0,
                                                int d0, half_t* const (&dst)[kMergeRows]) {
   constexpr int NR = kMergeRows;
-  constexpr int RG = kMergeRowStride;
+  constexpr int RG = kMergeRowStride<D>;
   constexpr int B = kMergeBatch;
   const float* wo = ws;
   const float* wml = ws + total_slots * slot_rows * D;
@@ -710,51 +784,56 @@ __device__ __forceinline__ void merge_partials(const float* __restrict__ ws, int
 }
 
 // Merge of the 4-wavefront tile kernel's split tiles (the mixed-step kernel's prefill part).
-// Grid (4 * tiles, P, H): workgroup (4 i + q) merges rows 32q .. 32q+31 of tile i if it was split;
-// partials are slot-major per (sequence, head), kTileRows rows per slot.
-template <int D>
+// Grid (parts * tiles, P, H), parts = kMergeParts<D, KS>: workgroup (parts i + q) merges the q-th part
+// of tile i's rows if it was split; partials are slot-major per (sequence, head), TR rows
+// per slot.
+template <int D, int KS>
 __device__ __forceinline__ void prefill_merge_body(
     const float* __restrict__ ws, half_t* __restrict__ out, int64_t o_st, int64_t num_tokens,
     int max_blocks, const int* __restrict__ seq_lens, const int* __restrict__ qsl,
-    int num_decode, int H, int smax, int slots, int P, int bx, int by, int bz, int tile_stride) {
+    int num_decode, int H, int smax, int slots, int P, int bx, int by, int bz, int tile_stride,
+    PrefillCaps caps) {
+  constexpr int TR = tile_rows(KS);
   constexpr int TPR = D / 8;                       // threads per row
-  constexpr int RG = kMergeRowStride;              // row groups per workgroup (16)
+  constexpr int RG = kMergeRowStride<D>;           // row groups per workgroup
   constexpr int NR = kMergeRows;                   // rows per thread
-  static_assert(RG * NR * 4 == kTileRows && TPR * RG == kTileThreads, "four workgroups per tile");
-  const int part = bx & 3;
+  constexpr int PARTS = kMergeParts<D, KS>;
+  static_assert(RG * NR * PARTS == TR && TPR * RG == kTileThreads, "whole parts per tile");
+  const int part = bx % PARTS;
   const int b = num_decode + by, h = bz;
-  const PrefillSeq sq = prefill_seq(qsl, seq_lens, b, num_tokens, max_blocks);
+  const PrefillSeq sq = prefill_seq(qsl, seq_lens, b, num_tokens, max_blocks, caps.rows);
+  if (sq.seq_len > caps.seq) return;               // its tiles ran unsplit
   const int rbase = part * RG * NR + (int)(threadIdx.x / TPR);   // rows rbase + RG * k
   const int d0 = 8 * (int)(threadIdx.x % TPR);
   const int64_t total = (int64_t)P * H * slots;
   // The grid covers the tiles the host bounds foresee; a sequence with more (bounds below its
   // real q_len) has its further tiles taken in turn, so every tile whose splits all ran is
   // merged (the tile kernel fills the rows of the others with NaN).
-  for (int tile = bx >> 2; tile * kTileRows < sq.q_len; tile += tile_stride) {
-    if (tile * kTileRows + rbase >= sq.q_len) continue;
-    const int2_t span = tile_span(tile, sq.q_len, sq.prefix, sq.seq_len, smax, kTileRows);
+  for (int tile = bx / PARTS; tile * TR < sq.q_len; tile += tile_stride) {
+    if (tile * TR + rbase >= sq.q_len) continue;
+    const int2_t span = tile_span(tile, sq.q_len, sq.prefix, sq.seq_len, smax, TR);
     const int slot = span[0], nsplit = span[1];
     if (nsplit <= 1 || slot + nsplit > slots) continue;   // unsplit, or splits past the launch
     half_t* dst[NR];
 #pragma unroll
     for (int k = 0; k < NR; ++k) {
-      const int row = tile * kTileRows + rbase + RG * k;
+      const int row = tile * TR + rbase + RG * k;
       dst[k] = row < sq.q_len ? out + (int64_t)(sq.q_start + row) * o_st + (int64_t)h * D + d0
                               : nullptr;
     }
-    merge_partials<D>(ws, total, kTileRows, ((int64_t)by * H + h) * slots + slot, nsplit, rbase,
+    merge_partials<D>(ws, total, TR, ((int64_t)by * H + h) * slots + slot, nsplit, rbase,
                       d0, dst);
   }
 }
 
-template <int D>
+template <int D, int KS>
 __global__ void __launch_bounds__(kTileThreads) prefill_merge_kernel(
     const float* __restrict__ ws, half_t* __restrict__ out, int64_t o_st, int64_t num_tokens,
     int max_blocks, const int* __restrict__ seq_lens, const int* __restrict__ qsl,
-    int num_decode, int H, int smax, int slots) {
-  prefill_merge_body<D>(ws, out, o_st, num_tokens, max_blocks, seq_lens, qsl, num_decode, H, smax,
+    int num_decode, int H, int smax, int slots, PrefillCaps caps) {
+  prefill_merge_body<D, KS>(ws, out, o_st, num_tokens, max_blocks, seq_lens, qsl, num_decode, H, smax,
                         slots, (int)gridDim.y, (int)blockIdx.x, (int)blockIdx.y,
-                        (int)blockIdx.z, (int)gridDim.x / 4);
+                        (int)blockIdx.z, (int)gridDim.x / kMergeParts<D, KS>, caps);
 }
 
 // Host-side plan of the 4-wavefront tiled path: the most steps one split may take (smax) and the
@@ -768,8 +847,9 @@ struct TilePlan {
 inline int cdiv(int a, int b) { return (a + b - 1) / b; }
 
 inline TilePlan tile_plan(int P, int H, int D, int max_query_len, int max_seq_len, int cu_count,
-                          bool split, int64_t round = 0) {
-  const int tiles = cdiv(max_query_len, kTileRows);
+                          bool split, int64_t round = 0, int tr = kTileRows,
+                          int min_steps = kPrefillMinSteps) {
+  const int tiles = cdiv(max_query_len, tr);
   const int seq = max_seq_len > max_query_len ? max_seq_len : max_query_len;
   const int nmax = cdiv(seq, kTileKeys);           // most steps any tile can have
   TilePlan pl{nmax > 0 ? nmax : 1, tiles, 0, (int64_t)tiles * P * H};
@@ -780,7 +860,7 @@ inline TilePlan tile_plan(int P, int H, int D, int max_query_len, int max_seq_le
   auto workgroups = [&](int smax) {
     int64_t n_wg = 0;
     for (int i = 0; i < tiles; ++i) {
-      const int hi = prefix + ((i + 1) * kTileRows < max_query_len ? (i + 1) * kTileRows : max_query_len);
+      const int hi = prefix + ((i + 1) * tr < max_query_len ? (i + 1) * tr : max_query_len);
       const int n = cdiv(hi, kTileKeys);
       n_wg += n <= smax ? 1 : cdiv(n, smax);
     }
@@ -792,13 +872,13 @@ inline TilePlan tile_plan(int P, int H, int D, int max_query_len, int max_seq_le
   // unsplit tiles already fill it, do not split.
   if (round <= 0) round = 2 * (int64_t)(cu_count > 0 ? cu_count : 256);
   if (workgroups(nmax) >= round) return pl;
-  int smax = kPrefillMinSteps;
+  int smax = min_steps;
   while (smax < nmax && workgroups(smax) > round) ++smax;
   if (smax >= nmax) return pl;
   pl.smax = smax;
   pl.est_wg = workgroups(smax);
   pl.slots = tiles * cdiv(nmax, smax);
-  pl.ws_bytes = (size_t)P * H * pl.slots * kTileRows * (D + 2) * sizeof(float);
+  pl.ws_bytes = (size_t)P * H * pl.slots * tr * (D + 2) * sizeof(float);
   return pl;
 }
 

@@ -485,7 +485,7 @@ __global__ void __launch_bounds__(kTileThreads) prefill_pair_merge_kernel(
     int num_decode, int H, int KVH, int slots, int seg_cap) {
   constexpr int D = PairLayout::D;
   constexpr int TPR = D / 8;
-  constexpr int RG = kMergeRowStride;
+  constexpr int RG = kMergeRowStride<128>;
   constexpr int NR = kMergeRows;
   static_assert(RG * NR * 4 == kTileRows && TPR * RG == kTileThreads, "four workgroups per block");
   const int bx = (int)blockIdx.x, by = (int)blockIdx.y, h = (int)blockIdx.z;

@@ -74,9 +74,9 @@ __global__ void __launch_bounds__(256, 2) ragged_split_kernel(const RaggedArgs a
   __shared__ __attribute__((aligned(16))) char lds[kRaggedLds];
   const int bx = (int)blockIdx.x;
   if (bx < a.pf_launch) {
-    prefill_tile_body<128>(a.q, a.q_st, a.q_sh, a.out, a.o_st, a.num_tokens, a.kc, a.vc, a.NB,
+    prefill_tile_body<128, 1>(a.q, a.q_st, a.q_sh, a.out, a.o_st, a.num_tokens, a.kc, a.vc, a.NB,
                            a.bt, a.bt_st, a.max_blocks, a.seq_lens, a.qsl, a.num_decode, a.H,
-                           a.KVH, a.sl2, a.smax, a.slots, a.P, a.pf_ws, bx, lds);
+                           a.KVH, a.sl2, a.smax, a.slots, a.P, kNoCaps, a.pf_ws, bx, lds);
   } else {
     // the decode splits run the LDS-ring form of decode_mfma_kernel: its two K slots fit in the
     // prefill tiles' LDS, the first one shared with the merge's LDS as there
@@ -98,9 +98,9 @@ __global__ void __launch_bounds__(256) ragged_merge_kernel(const RaggedArgs a) {
   } else {
     const int p = bx - a.dm_launch;
     const int x = p % a.pm_x, rest = p / a.pm_x;
-    prefill_merge_body<128>(a.pf_ws, a.out, a.o_st, a.num_tokens, a.max_blocks, a.seq_lens,
+    prefill_merge_body<128, 1>(a.pf_ws, a.out, a.o_st, a.num_tokens, a.max_blocks, a.seq_lens,
                             a.qsl, a.num_decode, a.H, a.smax, a.slots, a.P, x, rest % a.P,
-                            rest / a.P, a.pm_x / 4);
+                            rest / a.P, a.pm_x / kMergeParts<128, 1>, kNoCaps);
   }
 }
 
@@ -236,7 +236,7 @@ extern "C" int ts_paged_attention(const void* q, int64_t q_stride_t, int64_t q_s
       a.cap_blocks = r.dec.cap_blocks < max_blocks_per_seq ? r.dec.cap_blocks : max_blocks_per_seq;
       a.max_splits = r.dec.max_splits;
       a.dm_launch = num_decode * num_kv_heads * a.HG;
-      a.pm_x = 4 * cdiv(max_query_len, kTileRows);
+      a.pm_x = kMergeParts<128, 1> * cdiv(max_query_len, kTileRows);
       const hipStream_t s = reinterpret_cast<hipStream_t>(stream);
       const int n_split = a.pf_launch + a.nslots * num_kv_heads * a.HG;
       ragged_split_kernel<<<n_split, 256, 0, s>>>(a);
