@@ -26,6 +26,7 @@ typedef float float2_t __attribute__((ext_vector_type(2)));
 typedef float float4_t __attribute__((ext_vector_type(4)));
 typedef int int4_t __attribute__((ext_vector_type(4)));
 typedef int int2_t __attribute__((ext_vector_type(2)));
+typedef unsigned uint4_t __attribute__((ext_vector_type(4)));
 
 constexpr int kBlockSize = 16;    // tokens per KV block (config.py:74-75)
 constexpr int kWave = 64;         // CDNA wavefront width
@@ -56,6 +57,9 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t coherent_rsrc(const void* unif
 }
 __device__ __forceinline__ void coherent_store(__amdgpu_buffer_rsrc_t r, int off, float v) {
   __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, v), r, off, 0, kCoherentPolicy);
+}
+__device__ __forceinline__ void coherent_store4(__amdgpu_buffer_rsrc_t r, int off, float4_t v) {
+  __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(uint4_t, v), r, off, 0, kCoherentPolicy);
 }
 __device__ __forceinline__ float coherent_load(__amdgpu_buffer_rsrc_t r, int off) {
   return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, off, 0, kCoherentPolicy));
@@ -104,6 +108,11 @@ __device__ __forceinline__ int clamp_block(int blk, int64_t num_blocks) {
 // no restrict), so the entry does not wait behind the wavefront's vector loads.
 __device__ __forceinline__ int table_entry(const int* p) {
   return *reinterpret_cast<const __attribute__((address_space(4))) int*>(
+      reinterpret_cast<uintptr_t>(p));
+}
+
+__device__ __forceinline__ int64_t table_entry64(const int64_t* p) {
+  return *reinterpret_cast<const __attribute__((address_space(4))) int64_t*>(
       reinterpret_cast<uintptr_t>(p));
 }
 

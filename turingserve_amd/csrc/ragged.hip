@@ -86,7 +86,7 @@ __global__ void __launch_bounds__(256, 2) ragged_split_kernel(const RaggedArgs a
         a.q, a.q_st, a.q_sh, a.out, a.o_st, a.kc, a.vc, a.NB, a.bt, a.bt_st, a.max_blocks,
         a.seq_lens, a.num_decode, a.H, a.KVH, a.G, a.HG, a.sl2, a.cap_blocks, 0, a.max_splits,
         a.ws_acc, a.ws_m, a.ws_l, a.ws_cnt, d / (a.KVH * a.HG), d % (a.KVH * a.HG), lds,
-        NewRows{}, nullptr, 0, ring, ring + kRaggedRing1);
+        NewRows{}, nullptr, 0, nullptr, ring, ring + kRaggedRing1);
   }
 }
 
