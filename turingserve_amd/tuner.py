@@ -49,6 +49,9 @@ class VariantTable:
     def set(self, kernel: str, key, choice: dict) -> None:
         self._by_kernel.setdefault(kernel, {})[tuple(int(k) for k in key)] = dict(choice)
 
+    def empty(self, kernel: str) -> bool:
+        return not self._by_kernel.get(kernel)
+
     def records(self, kernel: str) -> dict[tuple[int, ...], dict]:
         return dict(self._by_kernel.get(kernel, {}))
 
@@ -94,6 +97,8 @@ def w8a16_choice(N: int, K: int, M: int) -> tuple[int, int]:
     smallest recorded M >= M (bisected over that shape's M list); else the library's own plan
     (0, 0). A streaming choice (variant 1) recorded for a bucket whose range reaches past
     M = 32 cannot apply and also falls back."""
+    if ACTIVE.empty("w8a16"):
+        return 0, 0
     shape = sorted((k[2], c) for k, c in ACTIVE.records("w8a16").items() if k[:2] == (N, K))
     i = bisect.bisect_left([m for m, _ in shape], M)
     if i == len(shape):
@@ -107,7 +112,7 @@ def w8a16_choice(N: int, K: int, M: int) -> tuple[int, int]:
 
 def decode_choice(S: int, max_seq_len: int) -> tuple[str | None, int | None]:
     """(version, partition) for S decode rows at this max_seq_len, or (None, None)."""
-    c = ACTIVE.lookup("decode", (S, max_seq_len))
+    c = None if ACTIVE.empty("decode") else ACTIVE.lookup("decode", (S, max_seq_len))
     if c is None:
         return None, None
     return c["version"], int(c["partition"])
