@@ -24,7 +24,12 @@ DEV = "cuda"
 TILES = [(1000, 15988, "256x256"), (575, 17884, "256x192"), (1790, 2004, "128x128 two K groups"),
          (1855, 1500, "128x96 four K groups"), (1000, 2004, "128x64 four K groups"),
          (750, 2004, "64x96 four K groups"), (67, 17884, "128x96 two K groups"),
-         (131, 17884, "128x64 two K groups")]
+         (131, 17884, "128x64 two K groups"), (9, 17884, "128x32 four K groups"),
+         (31, 17884, "128x32 four K groups")]
+# 64 x 32 tiles: products that the wide kernel would split over K (from K = 768 on), one of many
+# columns at long K, and at short K with fewer and more than 32 rows
+SMALL = [(47, 2004, "64x32", 768), (64, 1500, "64x32", 896), (20, 32996, "64x32", 3072),
+         (17, 9724, "64x32", 896), (63, 9724, "64x32", 128)]
 
 
 def _problem(M, N, Kd, fp16_scale=False):
@@ -37,8 +42,8 @@ def _problem(M, N, Kd, fp16_scale=False):
     return x, wq, scale, bias
 
 
-@pytest.mark.parametrize("Kd", [128, 384, 640])
-@pytest.mark.parametrize("M,N,tile", TILES)
+@pytest.mark.parametrize("M,N,tile,Kd", [(*t, k) for t in TILES for k in (128, 384, 640)] + SMALL +
+                         [(47, 2004, "64x32", 1152)])
 def test_every_tile_against_the_oracle(M, N, tile, Kd):
     x, wq, sc, bias = _problem(M, N, Kd, fp16_scale=Kd == 384)
     y = K.w8a16_linear(x.cuda(), wq.cuda(), sc.cuda(), bias.cuda()).float().cpu().numpy()
@@ -49,32 +54,33 @@ def test_every_tile_against_the_oracle(M, N, tile, Kd):
     assert (np.abs(y - ref.astype(np.float16).astype(np.float64)) <= ulp + 1e-4 * rms).all()
 
 
-@pytest.mark.parametrize("M,N,tile", TILES)
-def test_gated_epilogue_equals_the_pair(M, N, tile):
+@pytest.mark.parametrize("M,N,tile,Kd", [(*t, k) for t in TILES for k in (64, 256)] + SMALL)
+def test_gated_epilogue_equals_the_pair(M, N, tile, Kd):
     """The gated-MLP epilogue against the product then SiLU.up; also K of one 64-column step."""
     inter = N // 16 * 8                                       # the separate kernel needs I % 8 == 0
-    for Kd in (64, 256):
-        x, wq, sc, bias = (t.cuda() for t in _problem(M, 2 * inter, Kd))
-        fused = K.w8a16_glu(x, wq, sc, bias)
-        assert torch.equal(fused, K.silu_mul(K.w8a16_linear(x, wq, sc, bias)))
+    x, wq, sc, bias = (t.cuda() for t in _problem(M, 2 * inter, Kd))
+    fused = K.w8a16_glu(x, wq, sc, bias)
+    assert torch.equal(fused, K.silu_mul(K.w8a16_linear(x, wq, sc, bias)))
 
 
-@pytest.mark.parametrize("M,N,tile", TILES)
-def test_logits_epilogue_equals_the_gathered_product(M, N, tile):
-    x, wq, sc, _ = (t.cuda() for t in _problem(M, N, 256))
+@pytest.mark.parametrize("M,N,tile,Kd", [(*t, 256) for t in TILES] + SMALL)
+def test_logits_epilogue_equals_the_gathered_product(M, N, tile, Kd):
+    x, wq, sc, _ = (t.cuda() for t in _problem(M, N, Kd))
     rows = torch.randint(0, M, (M,), generator=torch.Generator().manual_seed(N)).cuda()
     got = K.logits_int8(x, rows, wq, sc)
     assert torch.equal(got, K.w8a16_linear(x[rows], wq, sc, None).float())
 
 
 @pytest.mark.parametrize("M,H,KVH", [(700, 12, 2), (1000, 12, 2), (1390, 12, 2), (1801, 12, 2),
-                                     (555, 100, 20), (1003, 84, 20)])
+                                     (555, 100, 20), (1003, 84, 20),
+                                     (20, 100, 20), (45, 12, 2), (64, 12, 2)])
 def test_rope_epilogue_equals_the_separate_calls(M, H, KVH):
     """Heads of 128 in tiles of 128 and 256 columns (700 rows: the plan's 64-column tile holds half
-    a head, so the fused call takes 128 columns), slots and positions out of range."""
+    a head, so the fused call takes 128 columns, as it does at 45 and 64 rows; at 20 the 128 x 32
+    tiles), slots and positions out of range."""
     from turingserve_amd.quant import LinearWeight
 
-    N, Kd, NB = (H + 2 * KVH) * 128, 256, 8 + M // 16
+    N, Kd, NB = (H + 2 * KVH) * 128, 256 if M > 64 else 1152, 8 + M // 16
     x, wq, sc, bias = (t.cuda() for t in _problem(M, N, Kd))
     g = torch.Generator().manual_seed(M)
     pos = torch.randint(-3, 600, (M,), generator=g).cuda()
@@ -89,3 +95,16 @@ def test_rope_epilogue_equals_the_separate_calls(M, H, KVH):
     qkv2 = K.w8a16_linear(x, wq, sc, bias)
     assert K.rope_kv_write_(qkv2, pos, cos, sin, H, KVH, 128, kv2[0], kv2[1], slots)
     assert torch.equal(qkv1, qkv2) and torch.equal(kv1, kv2)
+
+
+def test_weights_off_16_bytes_take_the_general_kernels():
+    """The block tiles' weight DMA wants 16-byte rows; 8-byte aligned weights are served by the wide
+    kernel, or, where that would split K (and the plan's workspace is none), by the skinny one."""
+    for M, N, Kd in ((47, 2048, 1536), (20, 17920, 256), (700, 2048, 256)):
+        x, wq, sc, bias = (t.cuda() for t in _problem(M, N, Kd))
+        off = torch.empty(N * Kd + 8, dtype=torch.int8, device=DEV)[8:].view(N, Kd).copy_(wq)
+        assert off.data_ptr() % 16 == 8
+        y = K.w8a16_linear(x, off, sc, bias).float().cpu().numpy()
+        ref = OQ.w8a16(x.cpu().numpy(), wq.cpu().numpy(), sc.cpu().numpy().astype(np.float64),
+                       bias.cpu().numpy(), np.float64)
+        assert np.linalg.norm(y - ref) / np.linalg.norm(ref) < 1e-3

@@ -1338,22 +1338,23 @@ static int wide64_splits(int M, int N, int K, int cus) {
   return splits;
 }
 
-// Block tiles (w8a16_tile_kernel) that replace a wide plan with one K split past M = 64; `rows` x
-// `cols` of Y^T, K steps of `bk`. The four with bk = 128 and four K groups sum K in the same order.
+// Block tiles (w8a16_tile_kernel), `rows` x `cols` of Y^T, K steps of `bk`. Those with four K groups
+// sum K in the same order.
 enum GemmTile : int {
   kTileNone = 0, kTile256x256, kTile256x192, kTile128x128k2, kTile128x96k4, kTile128x64k4,
-  kTile64x96k4, kTile128x96k2, kTile128x64k2
+  kTile64x96k4, kTile128x96k2, kTile128x64k2, kTile128x32k4, kTile64x32k4
 };
 struct TileSize { int rows, cols, bk; };
 constexpr TileSize kTileSizes[] = {{0, 0, 0},     {256, 256, 64}, {256, 192, 64},
                                    {128, 128, 128}, {128, 96, 128}, {128, 64, 128},
-                                   {64, 96, 128}, {128, 96, 64},  {128, 64, 64}};
+                                   {64, 96, 128}, {128, 96, 64},  {128, 64, 64},
+                                   {128, 32, 128}, {64, 32, 128}};
 static int64_t tile_count(int t, int M, int N) {
   const TileSize& s = kTileSizes[t];
   return (int64_t)((N + s.rows - 1) / s.rows) * ((M + s.cols - 1) / s.cols);
 }
 
-// Which block tile, for a product whose wide plan does not split K (measured with cold weights,
+// Which block tile past M = 64, for a product whose wide plan does not split K (cold weights,
 // wide plan -> block tile; one workgroup per CU unless said otherwise):
 //  * 256 x 256 or 256 x 192 where the output fills its resident rounds well enough that the
 //    larger operand blocks pay: at least 9/10 (16384 x 8192 at M = 2048: 620 -> 482 us) and 25/32
@@ -1389,6 +1390,31 @@ static int pick_tile(int M, int N, int K, int cus) {
   return kTileNone;
 }
 
+// Which block tile from M = 9 to 64, whose 32 rows leave the wide kernel's workgroups one MFMA per
+// operand read and too few bytes in flight (cold weights, plan below -> block tile):
+//  * 128 x 32 up to 32 rows while the tiles cover half the CUs (17920 x 1536, gated: M = 13 / 30
+//    13.5 / 13.8 -> 11.4 / 12.3 us), 64 x 32 past two of those per CU if K is long (37888 x 3584, gated:
+//    M = 13 / 30 42.9 / 46.8 -> 35.4 / 38.5 us, in place of streaming splits too; 151936 x 1536, with half
+//    the K steps to hide each tile's start and end behind, lost 2 to 6 % and stays);
+//  * 64 x 32 from 17 rows on at short K where they give half the CUs work and 128 x 32 tiles do not, or
+//    past 32 rows (9728 x 896, gated: M = 17 / 32 / 64 9.1 / 9.0 / 9.3 -> 6.6 / 6.5 / 8.1 us; up to 16
+//    rows the skinny kernel takes 6.5 to 7.1 us);
+//  * 64 x 32 for a product that would be split over K at short K, with no reduction launch: where the
+//    tiles reach a quarter of the CUs (2048 x 1536: M = 40 / 64 8.1 / 8.3 -> 6.9 / 7.0 us, with RoPE
+//    and the cache write 10.5 / 10.9 -> 8.5 / 8.6; 4608 x 3584 gained 1 us plain and lost as much with
+//    RoPE) or the split is two ways at most (1152 x 896: 7.7 -> 5.9 us; 896 x 896 with the norm that
+//    sums the partials: 8.8 -> 8.4). 1536 x 1536, 48 tiles, stays split: the norm reduces for nothing.
+static int pick_small_tile(int M, int N, int K, int cus, int splits) {
+  if (K % kTileSizes[kTile64x32k4].bk != 0 || M <= 8 || M > 64) return kTileNone;
+  const int64_t t64 = tile_count(kTile64x32k4, M, N), t128 = tile_count(kTile128x32k4, M, N);
+  const bool few_rows = M <= kSmallMMax;
+  if (t64 > 2LL * cus) return few_rows && K >= 3072 ? kTile64x32k4 : kTileNone;
+  if (splits > 1)
+    return !few_rows && K <= 2048 && (t64 * 4 >= cus || K <= 1024) ? kTile64x32k4 : kTileNone;
+  if (few_rows && t128 * 2 >= cus) return kTile128x32k4;
+  return M > 16 && K <= 2048 && t64 * 2 >= cus ? kTile64x32k4 : kTileNone;
+}
+
 // The plan of a variant with `splits` K splits (0: the variant's own rule). kVarAuto: weight
 // streaming when use_small_path says so; else 128 x 128 tiles (two workgroups per CU; the most
 // work per CU of the shapes measured) once they cover more than half the CUs and M is past 64
@@ -1402,9 +1428,7 @@ static int pick_tile(int M, int N, int K, int cus) {
 // cover under a quarter of the CUs, and unsplit for short-K products with many output channels
 // at M = 9 to 32 (use_wide32_wide_n). 128 x 32 tiles never split K by their own rule (splits 0),
 // and GLU mode plans them as 128 x 64.
-static GemmPlan plan_gemm_v(int M, int N, int K, int cus, int variant, int splits,
-                            bool glu = false) {
-  const bool own_rule = variant == kVarAuto;
+static GemmPlan plan_gemm_wide(int M, int N, int K, int cus, int variant, int splits, bool glu) {
   if (variant == kVarGemv || (variant == kVarAuto && use_gemv(M, N, K))) {
     GemmPlan p{false, 1, 0, 0, 1, K, 0, 0, 0, 0};
     gemv_shape(M, K, glu, &p);
@@ -1497,7 +1521,25 @@ static GemmPlan plan_gemm_v(int M, int N, int K, int cus, int variant, int split
     p.k_per_split = steps * kTileBK;
     p.splits = (K + p.k_per_split - 1) / p.k_per_split;
   }
-  if (own_rule && M > 64 && p.splits == 1) p.tile = pick_tile(M, N, K, cus);
+  return p;
+}
+
+// The plan above with a block tile in place of the wide, skinny or streaming kernel where the rules
+// of pick_tile and pick_small_tile say so.
+static GemmPlan plan_gemm_v(int M, int N, int K, int cus, int variant, int splits,
+                            bool glu = false) {
+  GemmPlan p = plan_gemm_wide(M, N, K, cus, variant, splits, glu);
+  if (variant != kVarAuto || p.gv > 0) return p;
+  if (M > 64) {
+    if (p.splits == 1) p.tile = pick_tile(M, N, K, cus);
+    return p;
+  }
+  const int t = pick_small_tile(M, N, K, cus, p.splits);
+  if (t != kTileNone) {
+    p.tile = t;
+    p.splits = 1;
+    p.k_per_split = K;
+  }
   return p;
 }
 
@@ -1548,6 +1590,11 @@ static int w8a16_launch(const half_t* xp, int64_t ldx, const int8_t* wq, const v
   if (p.gv > 0 && !(M <= kGemvMaxM && K % 16 == 0 && aligned(wq, 16) && aligned(xp, 16) &&
                     ldx % 8 == 0))
     p = plan_gemm_v(M, N, K, cus, kVarSkinny, 0, glu);   // the VALU path's alignment not met
+  if (p.tile != kTileNone && !aligned(wq, 16)) {  // the block tiles' weight DMA
+    p = plan_gemm_wide(M, N, K, cus, kVarAuto, 0, glu);
+    if (p.splits > 1)                             // the plan's size named no workspace
+      p = plan_gemm_wide(M, N, K, cus, kVarSkinny, 0, glu);
+  }
   if (glu && p.bm == 32) p.bm = 64;               // GLU tiles pair 32-row subtiles (same splits)
   const size_t need = gemm_workspace(p, M, N);
   TS_REQUIRE(need == 0 || (workspace && workspace_bytes >= need && aligned(workspace, 16)),
@@ -1566,6 +1613,38 @@ static int w8a16_launch(const half_t* xp, int64_t ldx, const int8_t* wq, const v
           part, p.splits, scale, scale_is_fp16, bp, yp, ldy, M, N, io);
     }
   };
+  if (p.tile != kTileNone) {
+    int t = p.tile;
+    // RoPE needs whole heads of 128 columns per tile (same K order, see GemmTile)
+    if (io.rope_cos && t == kTile64x96k4) t = kTile128x64k4;
+    if (io.rope_cos && t == kTile64x32k4) t = kTile128x32k4;
+    const TileSize& ts = kTileSizes[t];
+    const dim3 grid(glu ? (io.glu + ts.rows / 2 - 1) / (ts.rows / 2) : (N + ts.rows - 1) / ts.rows,
+                    (M + ts.cols - 1) / ts.cols);
+#define TS_TILE_CASE(ID, ...)                                                                      \
+  case ID: {                                                                                       \
+    using Shape = TileShape<__VA_ARGS__>;                                                          \
+    static_assert(Shape::kTN == kTileSizes[ID].rows && Shape::kTM == kTileSizes[ID].cols &&        \
+                  Shape::kBK == kTileSizes[ID].bk, "the planner's table");                         \
+    w8a16_tile_kernel<__VA_ARGS__><<<grid, Shape::kThreads, 0, s>>>(                               \
+        xp, ldx, wq, scale, scale_is_fp16, bp, yp, ldy, M, N, K, io);                              \
+    break;                                                                                         \
+  }
+    switch (t) {
+      TS_TILE_CASE(kTile256x256, 2, 4, 4, 2, 1, 1, 3)
+      TS_TILE_CASE(kTile256x192, 2, 3, 4, 2, 1, 1, 3)
+      TS_TILE_CASE(kTile128x128k2, 2, 2, 2, 2, 2, 2, 3)
+      TS_TILE_CASE(kTile128x96k4, 2, 3, 2, 1, 4, 2, 3)
+      TS_TILE_CASE(kTile128x64k4, 2, 2, 2, 1, 4, 2, 4)
+      TS_TILE_CASE(kTile64x96k4, 1, 3, 2, 1, 4, 2, 4)
+      TS_TILE_CASE(kTile128x96k2, 2, 3, 2, 1, 2, 1, 3)
+      TS_TILE_CASE(kTile128x64k2, 2, 2, 2, 1, 2, 1, 3)
+      TS_TILE_CASE(kTile128x32k4, 2, 1, 2, 1, 4, 2, 4)
+      TS_TILE_CASE(kTile64x32k4, 2, 1, 1, 1, 4, 2, 4)
+    }
+#undef TS_TILE_CASE
+    return TS_OK;
+  }
   if (p.gv > 0) {
     const int rows = 256 / p.gv * p.gvr;
     const dim3 grid(glu ? (io.glu + rows / 2 - 1) / (rows / 2) : (N + rows - 1) / rows);
@@ -1645,35 +1724,6 @@ static int w8a16_launch(const half_t* xp, int64_t ldx, const int8_t* wq, const v
   } else {
     float* part = p.splits > 1 ? static_cast<float*>(workspace) : nullptr;
     const bool fast = K % kTileBK == 0 && aligned(wq, 16);   // weight DMA, no K tail
-    if (p.tile != kTileNone && fast) {
-      int t = p.tile;
-      // RoPE needs whole heads of 128 columns per tile (same K order, see GemmTile)
-      if (io.rope_cos && t == kTile64x96k4) t = kTile128x64k4;
-      const TileSize& ts = kTileSizes[t];
-      const dim3 grid(glu ? (io.glu + ts.rows / 2 - 1) / (ts.rows / 2) : (N + ts.rows - 1) / ts.rows,
-                      (M + ts.cols - 1) / ts.cols);
-#define TS_TILE_CASE(ID, ...)                                                                      \
-  case ID: {                                                                                       \
-    using Shape = TileShape<__VA_ARGS__>;                                                          \
-    static_assert(Shape::kTN == kTileSizes[ID].rows && Shape::kTM == kTileSizes[ID].cols &&        \
-                  Shape::kBK == kTileSizes[ID].bk, "the planner's table");                         \
-    w8a16_tile_kernel<__VA_ARGS__><<<grid, Shape::kThreads, 0, s>>>(                               \
-        xp, ldx, wq, scale, scale_is_fp16, bp, yp, ldy, M, N, K, io);                              \
-    break;                                                                                         \
-  }
-      switch (t) {
-        TS_TILE_CASE(kTile256x256, 2, 4, 4, 2, 1, 1, 3)
-        TS_TILE_CASE(kTile256x192, 2, 3, 4, 2, 1, 1, 3)
-        TS_TILE_CASE(kTile128x128k2, 2, 2, 2, 2, 2, 2, 3)
-        TS_TILE_CASE(kTile128x96k4, 2, 3, 2, 1, 4, 2, 3)
-        TS_TILE_CASE(kTile128x64k4, 2, 2, 2, 1, 4, 2, 4)
-        TS_TILE_CASE(kTile64x96k4, 1, 3, 2, 1, 4, 2, 4)
-        TS_TILE_CASE(kTile128x96k2, 2, 3, 2, 1, 2, 1, 3)
-        TS_TILE_CASE(kTile128x64k2, 2, 2, 2, 1, 2, 1, 3)
-      }
-#undef TS_TILE_CASE
-      return TS_OK;
-    }
     const int tiles_n = glu ? (io.glu + p.bn / 2 - 1) / (p.bn / 2) : (N + p.bn - 1) / p.bn;
     const dim3 grid(tiles_n, (M + p.bm - 1) / p.bm, p.splits);
 #define TS_WIDE_LAUNCH(WNV, WMV)                                                                   \
