@@ -13,9 +13,28 @@ constexpr int kRowThreads = 256;
 constexpr int kRowVec = 8;                 // halves per 16-byte access
 constexpr int kRmsMaxIter = 4;             // N <= 4 * 256 * 8 = 8192
 
+template <int C>
+struct IntC { static constexpr int value = C; };
+
+// Sum over a wavefront, the same in every lane: the butterfly of lane xors 32, 16, 8, 4, 2, 1 on the
+// VALU (row and half-wave swaps, then DPP; a rotation by 4 of rows already equal 8 apart is the xor).
+__device__ __forceinline__ float wave_sum(float v) {
+  auto dpp = [](float x, auto ctrl) {
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), decltype(ctrl)::value, 0xf,
+                                                      0xf, true));
+  };
+  const auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  v = __uint_as_float(b[0]) + __uint_as_float(b[1]);
+  const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  v = __uint_as_float(a[0]) + __uint_as_float(a[1]);
+  v += dpp(v, IntC<0x128>{});                 // row_ror:8
+  v += dpp(v, IntC<0x124>{});                 // row_ror:4
+  v += dpp(v, IntC<0x4e>{});                  // quad_perm [2, 3, 0, 1]
+  return v + dpp(v, IntC<0xb1>{});            // quad_perm [1, 0, 3, 2]
+}
+
 __device__ __forceinline__ float block_sum_256(float v, float* s_red) {
-#pragma unroll
-  for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, kWave);
+  v = wave_sum(v);
   const int w = threadIdx.x / kWave, lane = threadIdx.x % kWave;
   if (lane == 0) s_red[w] = v;
   __syncthreads();
@@ -24,23 +43,34 @@ __device__ __forceinline__ float block_sum_256(float v, float* s_red) {
 
 // One row of N features by a workgroup of kRowThreads threads. load_x(i) returns features
 // i .. i+7 of the row's input; with kRes, res is added and the sum written to res_out.
+//
+// A row is a chain of load latencies (one workgroup per row, a few KB), so the residual and the
+// weight are requested together with the input: the weight's request used to wait for the sum of
+// squares, and the residual's for the reduction of a split product.
 template <bool kRes, class LoadX>
 __device__ __forceinline__ void rmsnorm_row(LoadX load_x, const half_t* __restrict__ res,
                                             const half_t* __restrict__ w, half_t* __restrict__ out,
                                             half_t* __restrict__ res_out, int N, float eps) {
   __shared__ float s_red[kRowThreads / kWave];
   const int tid = threadIdx.x;
-  half8_t v[kRmsMaxIter];
+  half8_t v[kRmsMaxIter], wv[kRmsMaxIter], rv[kRmsMaxIter];
   float ss = 0.f;
+#pragma unroll
+  for (int it = 0; it < kRmsMaxIter; ++it) {
+    const int i = (it * kRowThreads + tid) * kRowVec;
+    if (i < N) {
+      if constexpr (kRes) rv[it] = ld<half8_t>(res + i);
+      wv[it] = ld<half8_t>(w + i);
+    }
+  }
 #pragma unroll
   for (int it = 0; it < kRmsMaxIter; ++it) {
     const int i = (it * kRowThreads + tid) * kRowVec;
     if (i < N) {
       half8_t a = load_x(i);
       if constexpr (kRes) {
-        const half8_t b = ld<half8_t>(res + i);
 #pragma unroll
-        for (int e = 0; e < kRowVec; ++e) a[e] = (half_t)((float)a[e] + (float)b[e]);
+        for (int e = 0; e < kRowVec; ++e) a[e] = (half_t)((float)a[e] + (float)rv[it][e]);
         st<half8_t>(res_out + i, a);
       }
       v[it] = a;
@@ -53,12 +83,11 @@ __device__ __forceinline__ void rmsnorm_row(LoadX load_x, const half_t* __restri
   for (int it = 0; it < kRmsMaxIter; ++it) {
     const int i = (it * kRowThreads + tid) * kRowVec;
     if (i < N) {
-      const half8_t wv = ld<half8_t>(w + i);
       half8_t o;
 #pragma unroll
       for (int e = 0; e < kRowVec; ++e) {
         const half_t y = (half_t)((float)v[it][e] * inv);          // cast before the weight
-        o[e] = (half_t)((float)wv[e] * (float)y);
+        o[e] = (half_t)((float)wv[it][e] * (float)y);
       }
       st<half8_t>(out + i, o);
     }

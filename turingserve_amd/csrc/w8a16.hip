@@ -292,13 +292,19 @@ __global__ void __launch_bounds__(kSmWaves * 64) w8a16_small_kernel(
   }
 }
 
-// Output channel nn from its fp32 K sum: scale, bias, fp16.
+// Output channel from its fp32 K sum: scale, bias, fp16. The product is rounded before the bias is
+// added (no contraction), so that every kernel which sums partials gives the same value.
+__device__ __forceinline__ half_t finish_value(float s, float scale, bool has_bias, float bias) {
+#pragma clang fp contract(off)
+  float v = s * scale;
+  if (has_bias) v = v + bias;
+  return (half_t)v;
+}
 __device__ __forceinline__ half_t finish_channel(float s, const void* __restrict__ scale,
                                                  int scale_is_fp16, const half_t* __restrict__ bias,
                                                  int nn) {
-  float v = s * load_scale(scale, scale_is_fp16, nn);
-  if (bias) v += (float)bias[nn];
-  return (half_t)v;
+  return finish_value(s, load_scale(scale, scale_is_fp16, nn), bias != nullptr,
+                      bias ? (float)bias[nn] : 0.f);
 }
 
 // Element i of the [M, N] product from its split-K partials: sum (in split order), scale, bias,
@@ -367,19 +373,28 @@ __global__ void __launch_bounds__(kRowThreads) w8a16_reduce_rmsnorm_kernel(
   const int64_t t = blockIdx.x;
   const int64_t total = (int64_t)M * N;
   auto load_x = [&](int i) {
+    float sc[8], bs[8] = {};
+    if (scale_is_fp16) {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) sc[e] = (float)static_cast<const half_t*>(scale)[i + e];
+    } else {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) sc[e] = static_cast<const float*>(scale)[i + e];
+    }
+    if (bias) {
+#pragma unroll
+      for (int e = 0; e < 8; ++e) bs[e] = (float)bias[i + e];
+    }
     float4_t a = {0.f, 0.f, 0.f, 0.f}, b = {0.f, 0.f, 0.f, 0.f};
-    constexpr int U = 4;                         // partials requested before any is summed
-    for (int k0 = 0; k0 < splits; k0 += U) {
+    const float* row = part + t * N + i;
+    auto add = [&](auto u_, int k0) {            // U partials requested before any is summed
+      constexpr int U = decltype(u_)::value;
       float4_t va[U], vb[U];
 #pragma unroll
-      for (int u = 0; u < U; ++u) {
-        if (k0 + u < splits) {                   // uniform over the workgroup
-          const float* pp = part + (int64_t)(k0 + u) * total + t * N + i;
-          va[u] = ld<float4_t>(pp);
-          vb[u] = ld<float4_t>(pp + 4);
-        } else {
-          va[u] = vb[u] = float4_t{0.f, 0.f, 0.f, 0.f};
-        }
+      for (int u = 0; u < U; ++u) {              // past the last: the last once more, not added
+        const float* pp = row + (k0 + u < splits ? k0 + u : splits - 1) * total;
+        va[u] = ld<float4_t>(pp);
+        vb[u] = ld<float4_t>(pp + 4);
       }
 #pragma unroll
       for (int u = 0; u < U; ++u)
@@ -387,13 +402,16 @@ __global__ void __launch_bounds__(kRowThreads) w8a16_reduce_rmsnorm_kernel(
           a += va[u];
           b += vb[u];
         }
+    };
+    if (splits <= 4) {
+      add(IntC<4>{}, 0);
+    } else {
+      for (int k0 = 0; k0 < splits; k0 += 8) add(IntC<8>{}, k0);
     }
     half8_t v;
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      v[e] = finish_channel(a[e], scale, scale_is_fp16, bias, i + e);
-      v[4 + e] = finish_channel(b[e], scale, scale_is_fp16, bias, i + 4 + e);
-    }
+    for (int e = 0; e < 8; ++e)
+      v[e] = finish_value(e < 4 ? a[e] : b[e - 4], sc[e], bias != nullptr, bs[e]);
     return v;
   };
   rmsnorm_row<true>(load_x, res + t * res_st, w, out + t * out_st, res_out + t * res_out_st, N,
