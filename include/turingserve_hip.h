@@ -240,7 +240,7 @@ int ts_decode_rope_kv_write_attention(int32_t version, void* qkv, int64_t qkv_st
  * absolute position prefix + i, prefix = seq_lens[b] - q_len; it attends to keys
  * j <= prefix + i (bottom-right causal mask) read through block_tables[b].
  * num_tokens bounds every q / out row the kernel touches.
- * Without a workspace every 128-row query tile runs as one workgroup.
+ * Without a workspace every query tile runs as one workgroup.
  * Replaces ops/triton_prefill_attention.py:66-79.
  */
 int ts_prefill_attention(const void* q, int64_t q_stride_t, int64_t q_stride_h,
@@ -254,8 +254,8 @@ int ts_prefill_attention(const void* q, int64_t q_stride_t, int64_t q_stride_h,
 
 /*
  * The same with a workspace of ts_prefill_workspace_bytes() bytes (16-byte aligned): at
- * head_dim 128 the key range of a long query tile is then split over several workgroups whose
- * fp32 partials a merge kernel combines, so short chunks on long prefixes still fill the
+ * head_dim 64 and 128 the key range of a long query tile is then split over several workgroups whose
+ * partials a merge kernel combines, so short chunks on long prefixes still fill the
  * device. max_seq_len: a host-side upper bound of the prefill sequences' seq_lens. A smaller
  * workspace (or none) runs the tiles unsplit. Same results up to fp32 summation order.
  * Replaces ops/triton_prefill_attention.py:66-79 (the launch grid of :72-79).

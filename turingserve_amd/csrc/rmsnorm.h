@@ -13,7 +13,7 @@ constexpr int kRowThreads = 256;
 constexpr int kRowVec = 8;                 // halves per 16-byte access
 constexpr int kRmsMaxIter = 4;             // N <= 4 * 256 * 8 = 8192
 
-template <int C>
+template <int C>                           // an integer as a type, for the arguments of generic lambdas
 struct IntC { static constexpr int value = C; };
 
 // Sum over a wavefront, the same in every lane: the butterfly of lane xors 32, 16, 8, 4, 2, 1 on the
@@ -45,8 +45,9 @@ __device__ __forceinline__ float block_sum_256(float v, float* s_red) {
 // i .. i+7 of the row's input; with kRes, res is added and the sum written to res_out.
 //
 // A row is a chain of load latencies (one workgroup per row, a few KB), so the residual and the
-// weight are requested together with the input: the weight's request used to wait for the sum of
-// squares, and the residual's for the reduction of a split product.
+// weight are requested together with the input, not after the reduction of a split product and
+// after the sum of squares (a row of the M = 1 projections with the norm behind it: 1536 x 8960 8.0 ->
+// 7.9 us, 3584 x 18944 20.0 -> 19.7 us; 2048 rows of 8192 alone 25.7 -> 24.4 us).
 template <bool kRes, class LoadX>
 __device__ __forceinline__ void rmsnorm_row(LoadX load_x, const half_t* __restrict__ res,
                                             const half_t* __restrict__ w, half_t* __restrict__ out,

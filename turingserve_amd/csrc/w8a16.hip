@@ -12,10 +12,12 @@
 //    64-wide K step (64 bytes per row and instruction). The K dimension is split over
 //    workgroups until the device is full; fp32 partials are merged (and scaled) by a second
 //    kernel.
-//  * larger M: the wide-tile kernel on v_mfma_f32_32x32x16_f16 (128 x 128, 128 x 64 or 128 x 32 tiles of
-//    Y^T, split-K when the grid is short of two workgroups per CU): weights stream straight
-//    into the A operands of the wavefront that owns them, activations are DMA'd into a ring of
-//    LDS stages that all four wavefronts read.
+//  * larger M: the wide-tile kernel on v_mfma_f32_32x32x16_f16 (128 x 192, 128 x 128, 128 x 64 or 128 x 32
+//    tiles of Y^T, split-K when the grid is short of two workgroups per CU): weights and activations
+//    are DMA'd into a ring of LDS stages; each of four wavefronts owns 32 weight rows and reads every
+//    activation row.
+//  * from M = 9, where pick_tile and pick_small_tile say so: the block tiles of w8a16_tile.h, with larger
+//    operand blocks per wavefront, or K groups inside the workgroup in place of a K split.
 #include "common.h"
 #include "rmsnorm.h"
 #include "rope.h"
@@ -365,6 +367,13 @@ __global__ void __launch_bounds__(256) w8a16_glu_reduce_kernel(
 // a decoder layer): row t of y is reduced as w8a16_reduce_kernel reduces it (split order, scale,
 // bias, fp16), then res_out = y + res and out = rmsnorm(res_out) * w as the standalone norm
 // computes them, so the pair of launches replaces reduce + norm with the same values.
+// One workgroup per row, so load latency bounds it (a row of 8 splits is 49 KB, from the cache behind
+// all XCDs): scale, bias and up to 8 partials (all of them at the splits that the rules plan, or two
+// rounds) are requested before the first is used, behind rmsnorm_row's residual and weight. With four
+// at a time and the other operands after them, product and norm together took at 1536 x 8960
+// M = 16 / 32 / 64 12.5 / 13.7 / 14.9 -> 11.5 / 12.5 / 13.7 us, at 3584 x 3584 M = 32 / 64 14.5 / 16.1 ->
+// 12.6 / 15.1 us, at 896 x 4864 M = 64 11.0 -> 10.5 us. Up to 4 splits take batches of 4, which spare
+// the repeated requests of the last partial (1536 x 1536, 4 splits, M = 64: 9.4 -> 9.2 us).
 __global__ void __launch_bounds__(kRowThreads) w8a16_reduce_rmsnorm_kernel(
     const float* __restrict__ part, int splits, const void* __restrict__ scale, int scale_is_fp16,
     const half_t* __restrict__ bias, const half_t* __restrict__ res, int64_t res_st,

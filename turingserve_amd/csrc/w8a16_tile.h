@@ -1,5 +1,5 @@
-// W8A16 GEMM, block tiles (M > 64): wavefronts of 64 weight rows x 64 or 96 activation rows, and
-// K groups inside the workgroup. Included by w8a16.hip.
+// W8A16 GEMM, block tiles: wavefronts of up to 64 weight rows x 128 activation rows, and K groups
+// inside the workgroup. Included by w8a16.hip.
 #pragma once
 
 namespace ts {
