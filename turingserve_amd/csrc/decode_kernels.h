@@ -237,7 +237,7 @@ __device__ __forceinline__ int4 int4_of(int a, int b, int c, int d) { return int
 // Eight threads per launch slot, one 16-byte piece of its entry each (entries leave as whole
 // 128-byte lines, and a thread waits for at most four table entries); every workgroup computes
 // the prefix of the split counts for itself. One thread per slot over 3 workgroups took 8.8 us for
-// 64 sequences of up to 4096 tokens (704 slots), this form MAPNEW.
+// 64 sequences of up to 4096 tokens (704 slots), this form 4.7 us.
 template <int NT>
 __global__ void __launch_bounds__(NT) decode_split_map_kernel(
     const int* __restrict__ seq_lens, const int* __restrict__ bt, int64_t bt_st, int64_t NB,
@@ -447,7 +447,6 @@ __device__ __forceinline__ void decode_mfma_body(
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int c = lane & 15, g = lane >> 4;
   const int hq = hg * 16 + c;                    // query head within the GQA group
-  const bool head_ok = hq < G;
   const int nh = (G - hg * 16) < 16 ? (G - hg * 16) : 16;   // real heads in this group
   const int head0 = kvh * G + hg * 16;           // first query head of this group
   const bool split = ws_acc != nullptr;
@@ -463,9 +462,9 @@ __device__ __forceinline__ void decode_mfma_body(
   if constexpr (2 * NW == kMapPairs) {
     if (split && smap != nullptr) {
       const int* e = smap + kMapHeader + (int64_t)bx * kMapEntry;
-      mapped = smap[0] == kMapMagic && smap[1] == S && smap[2] == nslots &&
-               smap[3] == part_blocks && smap[5] == max_splits &&
-               smap[6] == cap_blocks;
+      // (no short circuit: each would wait for its own load of the header's line)
+      mapped = ((smap[0] ^ kMapMagic) | (smap[1] ^ S) | (smap[2] ^ nslots) |
+                (smap[3] ^ part_blocks) | (smap[5] ^ max_splits) | (smap[6] ^ cap_blocks)) == 0;
       sp = {e[0], e[1], e[2], e[7], e[3]};
       m_last = e[6];
       m_id[0] = e[8 + 2 * w];
@@ -538,15 +537,17 @@ __device__ __forceinline__ void decode_mfma_body(
     return clamp_block(table_entry(btrow + bi), NB);
   };
 
+  // Lanes past the group's heads read its last head: their columns of S^T and O^T are not used, and
+  // a masked load would be waited for before the first K/V request.
   half8_t qf[KK];
   {
-    const half_t* qp = q + (int64_t)s * q_st + (int64_t)(kvh * G + hq) * q_sh;
+    const half_t* qp = q + (int64_t)s * q_st + (int64_t)(kvh * G + (hq < G ? hq : G - 1)) * q_sh;
 #pragma unroll
     for (int kk = 0; kk < KK; ++kk) {
       if constexpr (D >= 32) {
-        qf[kk] = head_ok ? ld<half8_t>(qp + 32 * kk + 8 * g) : half8_t{0, 0, 0, 0, 0, 0, 0, 0};
+        qf[kk] = ld<half8_t>(qp + 32 * kk + 8 * g);
       } else {
-        const half4_t t = head_ok ? ld<half4_t>(qp + 4 * g) : half4_t{0, 0, 0, 0};
+        const half4_t t = ld<half4_t>(qp + 4 * g);
         qf[kk] = {t[0], t[1], t[2], t[3], 0, 0, 0, 0};
       }
     }
@@ -598,7 +599,7 @@ __device__ __forceinline__ void decode_mfma_body(
   float4_t cs[ROPE ? KK / 2 : 1][2], sn[ROPE ? KK / 2 : 1][2];
   constexpr int PIECES = D / 8;                  // 16-byte pieces per row
   constexpr int PK = ROPE ? D / 16 : PIECES;     // threads writing K (with RoPE: 8 frequencies)
-  half8_t x1 = {}, x2 = {};                      // the new row's pieces of this thread
+  half8_t x1, x2;                                // the new row's pieces of this thread
   float4_t wc[2], ws[2];
   auto request_tables = [&](int64_t row) {
     if constexpr (ROPE) {
@@ -611,11 +612,11 @@ __device__ __forceinline__ void decode_mfma_body(
           cs[kk][e] = ld<float4_t>(ct + 32 * kk + 8 * g + 4 * e);
           sn[kk][e] = ld<float4_t>(st + 32 * kk + 8 * g + 4 * e);
         }
-      if (ends && tid < PK) {
+      if (ends) {                                // every thread, as in request_rows
 #pragma unroll
         for (int e = 0; e < 2; ++e) {
-          wc[e] = ld<float4_t>(ct + 8 * tid + 4 * e);
-          ws[e] = ld<float4_t>(st + 8 * tid + 4 * e);
+          wc[e] = ld<float4_t>(ct + 8 * (tid % PK) + 4 * e);
+          ws[e] = ld<float4_t>(st + 8 * (tid % PK) + 4 * e);
         }
       }
     }
@@ -626,13 +627,15 @@ __device__ __forceinline__ void decode_mfma_body(
     if (ends) {
       const half_t* ksrc = nr.k + (int64_t)s * nr.k_st + (int64_t)kvh * nr.k_sh;
       const half_t* vsrc = nr.v + (int64_t)s * nr.v_st + (int64_t)kvh * nr.v_sh;
-      if (tid < PK) {
-        // with RoPE frequencies 8 tid .. 8 tid + 7: dims of the first half and of the second
-        x1 = ld<half8_t>(ksrc + 8 * tid);
-        if constexpr (ROPE) x2 = ld<half8_t>(ksrc + D / 2 + 8 * tid);
-      } else if (tid < PK + PIECES) {
-        x1 = ld<half8_t>(vsrc + 8 * (tid - PK));
-      }
+      // K pieces (with RoPE frequencies 8 tid .. 8 tid + 7: dims of the first half and of the
+      // second), then V pieces. Every thread loads some piece: loads under divergent branches
+      // were waited for where the branches join, before the first V request (two layers of eight
+      // sequences of up to 300 tokens, 8/8 heads of 64, with q's unmasked load and the header's line
+      // read at once: 24.8 -> 23.9 us; 24 up to 8192, 14/2 of 64, eight layers 137.1 -> 124.5; 64 up
+      // to 4096, 12/2 of 128, four layers 103.7 -> 101.4).
+      const half_t* src = tid < PK ? ksrc + 8 * tid : vsrc + 8 * ((tid - PK) % PIECES);
+      x1 = ld<half8_t>(src);
+      if constexpr (ROPE) x2 = ld<half8_t>(tid < PK ? src + D / 2 : src);
     }
   };
   // q rotated in registers, as rope_kernel rotates it in memory: lane (c, g) holds dims
@@ -642,7 +645,10 @@ __device__ __forceinline__ void decode_mfma_body(
     if constexpr (ROPE) {
       static_assert(KK % 2 == 0, "RoPE pairs must sit in one lane (head_dim a multiple of 64)");
       const int64_t row = rope_row(pos, nr.max_pos);
-      if (row != likely_row) request_tables(row);
+      if (row != likely_row) {
+        request_tables(row);
+        __builtin_amdgcn_s_waitcnt(kWaitVmcntZero);   // here, not for both paths where they join
+      }
 #pragma unroll
       for (int kk = 0; kk < KK / 2; ++kk) {
         half4_t o1a, o2a, o1b, o2b;
@@ -827,6 +833,8 @@ __device__ __forceinline__ void decode_mfma_body(
       ids_of(last_or(p + 2 * NW, last_or(p + NW, p)), idn);
     } else {
       request_rows();
+      // pending loads of this path would be waited for where the paths join
+      __builtin_amdgcn_s_waitcnt(kWaitVmcntZero);
     }
     rotate_and_write();
     // The loop sits on the prologue's path only, so the compiler's wait state at its head is the
@@ -920,6 +928,8 @@ __device__ __forceinline__ void decode_mfma_body(
       ids_of(last_or(p + 2 * NW, last_or(p + NW, p)), idv);
     } else {
       request_rows();
+      // pending loads of this path would be waited for where the paths join
+      __builtin_amdgcn_s_waitcnt(kWaitVmcntZero);
     }
     rotate_and_write();
     if (mapped) poison = poison || stale();
