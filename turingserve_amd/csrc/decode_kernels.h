@@ -421,6 +421,13 @@ struct NewRows {
   int64_t qkv_st;
 };
 
+// A step of a wavefront's pairs: one with a pair two steps on, which it requests; the last but one, or
+// a wavefront's only one; or the last of several. Only the latter two can hold the range's last
+// pair (the mask, the new row).
+enum DecodeStep { kLoop, kLastButOne, kLast };
+template <DecodeStep S>
+using Left = std::integral_constant<int, S>;
+
 template <int D, int NW, bool WRITE = false, bool ROPE = false, bool KDMA = false>
 __device__ __forceinline__ void decode_mfma_body(
     const half_t* __restrict__ q, int64_t q_st, int64_t q_sh, half_t* __restrict__ out,
@@ -516,11 +523,8 @@ __device__ __forceinline__ void decode_mfma_body(
   // kv_write of sequence s's new row (ops/reference.py:50-57) for this KV head, by the workgroup
   // whose range ends the sequence (it holds position seq_len - 1, where every input builder puts
   // slot_mapping[s]; the launch has one head group per KV head, so no other workgroup reads that
-  // block). The row goes to the cache for later launches and to LDS for this one: the wavefront
-  // that takes the range's last pair puts it in place of the block's old row (patch_*), so no K/V
-  // request waits for the store (the earlier form stored, waited for the store and passed a barrier
-  // before any request; with q's rotation and the tables' row also off that path the launch of 64
-  // sequences took 25.3 -> 24.1 us, of one 13.0 -> 12.0, of four up to 32768 tokens 25.9 -> 24.0).
+  // block). The wavefront that takes the range's last pair puts the row in place of the block's old
+  // one (take_new_row) and stores it, so no K/V request waits for the store.
   bool fresh = false;                            // this workgroup writes the row
   const bool ends = WRITE && split_j == nsplit - 1;   // this range ends the sequence
   int64_t slot = -1, pos = 0;
@@ -560,15 +564,26 @@ __device__ __forceinline__ void decode_mfma_body(
 
   const int64_t head_off = (int64_t)kvh * kBlockSize * D;
   const int64_t blk_stride = (int64_t)KVH * kBlockSize * D;
-  // Two pipelines. KDMA (decode_mfma_kernel at D = 128, and the ragged launch): K of two pairs in a per-wavefront LDS ring filled by LDS DMA, V of two pairs in registers, so
-  // each pair's K and V are requested two pairs ahead. Otherwise: K of one pair in registers
-  // (refilled for the next pair as soon as the S^T MFMAs have consumed it) and V of two pairs
-  // (the next pair's V is requested a whole iteration before its P.V product). Either form keeps
-  // the kernel at two wavefronts per SIMD at D = 128; the remaining latency is hidden by the
-  // other resident wavefronts. The refills are unconditional (past a wavefront's last pair they
-  // repeat its current pair, a cache hit) so every iteration has the same loads in flight and
-  // each wait covers exactly what it needs. Block-table entries are scalar loads issued two
-  // pairs ahead.
+  // Two pipelines. KDMA (decode_mfma_kernel at D = 128, and the ragged launch): K of two pairs in a
+  // per-wavefront LDS ring filled by LDS DMA, V of two pairs in registers, so each pair's K and V
+  // are requested two pairs ahead. Otherwise: K of one pair in registers (refilled for the next pair
+  // as soon as the S^T MFMAs have consumed it) and V of two pairs (the next pair's V is requested a
+  // whole iteration before its P.V product). Either form keeps the kernel at two wavefronts per SIMD
+  // at D = 128; the remaining latency is hidden by the other resident wavefronts. Block-table entries
+  // are scalar loads issued two pairs ahead.
+  //
+  // A wavefront with a pair runs from its requests to its last step on a path of its own, and its loop
+  // holds only steps whose refills are used (Left): every iteration has the same loads in flight and
+  // each wait covers what it needs and no more. Where that path met another (wavefronts without a
+  // pair, a step with the mask or the new row, the loop left after its first step), the compiler
+  // waited for whichever side needed more: for the V rows of both pairs before q's rotation, and in
+  // the launches that do not write for the whole next pair in every second step. Two layers and the
+  // split map, in us, in that form -> in this one, with the new row left to its own wavefront: 8
+  // sequences of up to 300 tokens on 8/8 heads of 64 24.3 -> 20.7, 24 up to 8192 on 14/2 of 64 36.1 ->
+  // 33.0, 64 up to 2000 on 12/2 of 128 43.1 -> 40.8, 24 up to 8192 on 28/4 of 128 63.0 -> 57.7; the
+  // one-launch step of 48 up to 4096 and a 512-token chunk on 12/2 of 128 55.3 -> 51.6. (In a loop
+  // that takes every pair but the last two, whose last refill may repeat a pair, the 28/4 batch took
+  // 65.1: at the schedule's 24 blocks a wavefront has three pairs, and that refill is a third more.)
   auto load_k = [&](const int (&id)[2], half8_t (&kf)[2][KK]) {
 #pragma unroll
     for (int j = 0; j < 2; ++j) load_k_block<D>(kc + id[j] * blk_stride + head_off, c, g, kf[j]);
@@ -593,14 +608,16 @@ __device__ __forceinline__ void decode_mfma_body(
     const int cur_last = clamp_block(table_entry(btrow + (seq_len - 1) / kBlockSize), NB);
     return cur != seq_len || cur_last != m_last;
   };
-  // The RoPE tables' values for this lane's dims and the new row's pieces, requested between the
-  // first K and V loads. The tables are read at the row of position seq_len - 1, which every input
-  // builder passes, without waiting for positions[s]; another position is read again below.
+  // The wavefront that takes the range's last pair, alone, fetches the new row in the layouts of its
+  // operands (K as q, V as a token row), rotates K as it rotates q and keeps both in s_new, where only
+  // it reads them: no other wavefront loads more or waits at a barrier.
+  const bool owner = ends && w == (npairs - 1) % NW;
+  // The RoPE tables' values for this lane's dims. They are read at the row of position seq_len - 1,
+  // which every input builder passes, without waiting for positions[s]; another position is read
+  // again below.
   float4_t cs[ROPE ? KK / 2 : 1][2], sn[ROPE ? KK / 2 : 1][2];
-  constexpr int PIECES = D / 8;                  // 16-byte pieces per row
-  constexpr int PK = ROPE ? D / 16 : PIECES;     // threads writing K (with RoPE: 8 frequencies)
-  half8_t x1, x2;                                // the new row's pieces of this thread
-  float4_t wc[2], ws[2];
+  half8_t xk[KK];
+  VRow xv;
   auto request_tables = [&](int64_t row) {
     if constexpr (ROPE) {
       const float* ct = nr.cos_t + row * (D / 2);
@@ -612,129 +629,117 @@ __device__ __forceinline__ void decode_mfma_body(
           cs[kk][e] = ld<float4_t>(ct + 32 * kk + 8 * g + 4 * e);
           sn[kk][e] = ld<float4_t>(st + 32 * kk + 8 * g + 4 * e);
         }
-      if (ends) {                                // every thread, as in request_rows
-#pragma unroll
-        for (int e = 0; e < 2; ++e) {
-          wc[e] = ld<float4_t>(ct + 8 * (tid % PK) + 4 * e);
-          ws[e] = ld<float4_t>(st + 8 * (tid % PK) + 4 * e);
-        }
-      }
     }
   };
   const int64_t likely_row = ROPE ? rope_row(seq_len - 1, nr.max_pos) : 0;
   auto request_rows = [&]() {
     request_tables(likely_row);
-    if (ends) {
+    if (owner) {
       const half_t* ksrc = nr.k + (int64_t)s * nr.k_st + (int64_t)kvh * nr.k_sh;
       const half_t* vsrc = nr.v + (int64_t)s * nr.v_st + (int64_t)kvh * nr.v_sh;
-      // K pieces (with RoPE frequencies 8 tid .. 8 tid + 7: dims of the first half and of the
-      // second), then V pieces. Every thread loads some piece: loads under divergent branches
-      // were waited for where the branches join, before the first V request (two layers of eight
-      // sequences of up to 300 tokens, 8/8 heads of 64, with q's unmasked load and the header's line
-      // read at once: 24.8 -> 23.9 us; 24 up to 8192, 14/2 of 64, eight layers 137.1 -> 124.5; 64 up
-      // to 4096, 12/2 of 128, four layers 103.7 -> 101.4).
-      const half_t* src = tid < PK ? ksrc + 8 * tid : vsrc + 8 * ((tid - PK) % PIECES);
-      x1 = ld<half8_t>(src);
-      if constexpr (ROPE) x2 = ld<half8_t>(tid < PK ? src + D / 2 : src);
+      load_k_block<D>(ksrc, 0, g, xk);
+      if constexpr (VW == 1) {
+        xv = half2_t{vsrc[c], (half_t)0.f};
+      } else {
+        xv = ld<VRow>(vsrc + VW * c);
+      }
     }
   };
-  // q rotated in registers, as rope_kernel rotates it in memory: lane (c, g) holds dims
-  // 32 kk + 8 g .. + 7, and dims d and d + D / 2 (kk and kk + KK / 2) are a rotation pair. The new
-  // row, rotated as rope_kv_write_kernel rotates it, goes to the cache and to s_new.
-  auto rotate_and_write = [&]() {
+  // Rotated in registers, as rope_kernel and rope_kv_write_kernel rotate in memory: lane (c, g) holds
+  // dims 32 kk + 8 g .. + 7, and dims d and d + D / 2 (kk and kk + KK / 2) are a rotation pair.
+  auto rotate = [&](half8_t (&x)[KK]) {
     if constexpr (ROPE) {
       static_assert(KK % 2 == 0, "RoPE pairs must sit in one lane (head_dim a multiple of 64)");
+#pragma unroll
+      for (int kk = 0; kk < KK / 2; ++kk) {
+        half4_t o1a, o2a, o1b, o2b;
+        rope4(lo4(x[kk]), lo4(x[kk + KK / 2]), cs[kk][0], sn[kk][0], o1a, o2a);
+        rope4(hi4(x[kk]), hi4(x[kk + KK / 2]), cs[kk][1], sn[kk][1], o1b, o2b);
+        x[kk] = half8_t{o1a[0], o1a[1], o1a[2], o1a[3], o1b[0], o1b[1], o1b[2], o1b[3]};
+        x[kk + KK / 2] = half8_t{o2a[0], o2a[1], o2a[2], o2a[3], o2b[0], o2b[1], o2b[2], o2b[3]};
+      }
+    }
+  };
+  constexpr int PIECES = D / 8;                  // 16-byte pieces per row
+  auto rotate_rows = [&]() {
+    if constexpr (ROPE) {
       const int64_t row = rope_row(pos, nr.max_pos);
       if (row != likely_row) {
         request_tables(row);
         __builtin_amdgcn_s_waitcnt(kWaitVmcntZero);   // here, not for both paths where they join
       }
-#pragma unroll
-      for (int kk = 0; kk < KK / 2; ++kk) {
-        half4_t o1a, o2a, o1b, o2b;
-        rope4(lo4(qf[kk]), lo4(qf[kk + KK / 2]), cs[kk][0], sn[kk][0], o1a, o2a);
-        rope4(hi4(qf[kk]), hi4(qf[kk + KK / 2]), cs[kk][1], sn[kk][1], o1b, o2b);
-        qf[kk] = half8_t{o1a[0], o1a[1], o1a[2], o1a[3], o1b[0], o1b[1], o1b[2], o1b[3]};
-        qf[kk + KK / 2] = half8_t{o2a[0], o2a[1], o2a[2], o2a[3], o2b[0], o2b[1], o2b[2], o2b[3]};
-      }
+      rotate(qf);
     }
-    if (ends) {                                  // uniform over the workgroup
-      // The precondition of the fusion: the slot is that of position seq_len - 1. Any other slot
-      // would put the row in a block another workgroup may be reading; it is not written, and
-      // the sequence's output becomes NaN so the caller sees the broken precondition.
-      const int last_blk =
-          mapped ? m_last : clamp_block(table_entry(btrow + (seq_len - 1) / kBlockSize), NB);
-      const int64_t want = (int64_t)last_blk * kBlockSize + (seq_len - 1) % kBlockSize;
-      const bool in_cache = slot >= 0 && slot < nr.num_slots;
-      poison = in_cache && slot != want;
-      fresh = in_cache && !poison;
-      if (fresh) {
-        const int64_t row = (((slot >> 4) * KVH + kvh) * kBlockSize + (slot & 15)) * D;
-        half_t* krow = const_cast<half_t*>(kc) + row;
-        half_t* vrow = const_cast<half_t*>(vc) + row;
-        if (tid < PK) {
-          if constexpr (ROPE) {
-            half4_t o1a, o2a, o1b, o2b;
-            rope4(lo4(x1), lo4(x2), wc[0], ws[0], o1a, o2a);
-            rope4(hi4(x1), hi4(x2), wc[1], ws[1], o1b, o2b);
-            const half8_t y1 = {o1a[0], o1a[1], o1a[2], o1a[3], o1b[0], o1b[1], o1b[2], o1b[3]};
-            const half8_t y2 = {o2a[0], o2a[1], o2a[2], o2a[3], o2b[0], o2b[1], o2b[2], o2b[3]};
-            st<half8_t>(krow + 8 * tid, y1);
-            st<half8_t>(krow + D / 2 + 8 * tid, y2);
-            s_new[tid] = y1;
-            s_new[PK + tid] = y2;
-          } else {
-            st<half8_t>(krow + 8 * tid, x1);
-            s_new[tid] = x1;
-          }
-        } else if (tid < PK + PIECES) {
-          st<half8_t>(vrow + 8 * (tid - PK), x1);
-          s_new[PIECES + tid - PK] = x1;
+    if (owner) {
+      rotate(xk);
+#pragma unroll
+      for (int kk = 0; kk < KK; ++kk) {
+        if constexpr (D >= 32) {
+          s_new[4 * kk + g] = xk[kk];
+        } else {
+          reinterpret_cast<half4_t*>(s_new)[g] = lo4(xk[kk]);
         }
-        // s_new is published without waiting for the K/V requests in flight, as __syncthreads
-        // would
-        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+      }
+      if constexpr (VW == 1) {
+        reinterpret_cast<half_t*>(s_new + PIECES)[c] = xv[0];
+      } else {
+        *(reinterpret_cast<VRow*>(s_new + PIECES) + c) = xv;
       }
     }
   };
-  // The new row in place of row c_new of block j_new of the range's last pair.
-  const int c_new = (seq_len - 1) % kBlockSize;
-  const int j_new = ((seq_len - 1) / kBlockSize - blk_lo) & 1;
+  // The precondition of the fusion: the slot is that of position seq_len - 1. Any other slot would put
+  // the row in a block another workgroup may be reading; it is not written, and the sequence's
+  // output becomes NaN so the caller sees the broken precondition.
+  auto check_slot = [&]() {
+    if (!ends) return;                           // uniform over the workgroup
+    const int last_blk =
+        mapped ? m_last : clamp_block(table_entry(btrow + (seq_len - 1) / kBlockSize), NB);
+    const int64_t want = (int64_t)last_blk * kBlockSize + (seq_len - 1) % kBlockSize;
+    const bool in_cache = slot >= 0 && slot < nr.num_slots;
+    poison = in_cache && slot != want;
+    fresh = in_cache && !poison;
+  };
+  // The range's last pair: the new row in place of row c_new of block j_new, and to the cache.
+  const int c_new = (seq_len - 1) & (kBlockSize - 1);
+  const int j_new = (((seq_len - 1) / kBlockSize) ^ blk_lo) & 1;
+  const int k_at = c == c_new ? j_new : -1;      // this lane's operand rows that hold it
+  const int v_at = g == c_new >> 2 ? 4 * j_new + (c_new & 3) : -1;
   auto newest = [&](int p) { return WRITE && fresh && p == npairs - 1; };
-  auto patch_v = [&](VRow (&vr)[2][4]) {
-    if constexpr (WRITE && VW >= 2) {
-      const VRow nv = *(reinterpret_cast<const VRow*>(s_new + PIECES) + c);
-#pragma unroll
-      for (int j = 0; j < 2; ++j)
-#pragma unroll
-        for (int r = 0; r < 4; ++r)
-          if (j == j_new && r == c_new % 4) vr[j][r] = g == c_new / 4 ? nv : vr[j][r];
-    } else if constexpr (WRITE) {
-      const half_t nv = reinterpret_cast<const half_t*>(s_new + PIECES)[c];
-#pragma unroll
-      for (int j = 0; j < 2; ++j)
-#pragma unroll
-        for (int r = 0; r < 4; ++r)
-          if (j == j_new && r == c_new % 4) vr[j][r][0] = g == c_new / 4 ? nv : vr[j][r][0];
-    }
-  };
-  auto patch_k = [&](half8_t (&kf)[2][KK]) {
+  auto take_new_row = [&](half8_t (&kf)[2][KK], VRow (&vr)[2][4]) {
     if constexpr (WRITE) {
+      const int64_t row = (((slot >> 4) * KVH + kvh) * kBlockSize + (slot & 15)) * D;
+      half_t* krow = const_cast<half_t*>(kc) + row;
+      half_t* vrow = const_cast<half_t*>(vc) + row;
+#pragma unroll
+      for (int kk = 0; kk < KK; ++kk) {
+        if constexpr (D >= 32) {
+          const half8_t nk = s_new[4 * kk + g];
+#pragma unroll
+          for (int j = 0; j < 2; ++j) kf[j][kk] = k_at == j ? nk : kf[j][kk];
+          st<half8_t>(krow + 32 * kk + 8 * g, nk);
+        } else {
+          const half4_t nk = reinterpret_cast<const half4_t*>(s_new)[g];
+          const half8_t n8 = {nk[0], nk[1], nk[2], nk[3], 0, 0, 0, 0};
+#pragma unroll
+          for (int j = 0; j < 2; ++j) kf[j][kk] = k_at == j ? n8 : kf[j][kk];
+          st<half4_t>(krow + 4 * g, nk);
+        }
+      }
+      VRow nv;
+      if constexpr (VW == 1) {
+        nv = half2_t{reinterpret_cast<const half_t*>(s_new + PIECES)[c], (half_t)0.f};
+      } else {
+        nv = *(reinterpret_cast<const VRow*>(s_new + PIECES) + c);
+      }
 #pragma unroll
       for (int j = 0; j < 2; ++j)
-        if (j == j_new) {
 #pragma unroll
-          for (int kk = 0; kk < KK; ++kk) {
-            if constexpr (D >= 32) {
-              const half8_t nk = s_new[4 * kk + g];
-              kf[j][kk] = c == c_new ? nk : kf[j][kk];
-            } else {
-              const half4_t nk = reinterpret_cast<const half4_t*>(s_new)[g];
-              const half8_t n8 = {nk[0], nk[1], nk[2], nk[3], 0, 0, 0, 0};
-              kf[j][kk] = c == c_new ? n8 : kf[j][kk];
-            }
-          }
-        }
+        for (int r = 0; r < 4; ++r) vr[j][r] = v_at == 4 * j + r ? nv : vr[j][r];
+      if constexpr (VW == 1) {
+        vrow[c] = nv[0];
+      } else {
+        st<VRow>(vrow + VW * c, nv);
+      }
     }
   };
   if constexpr (KDMA) {
@@ -749,8 +754,9 @@ __device__ __forceinline__ void decode_mfma_body(
     // would drain every load in flight before any LDS read after an LDS DMA in a loop); their
     // waits are written out: each K pair's eight DMAs are followed, before the pair is read, by
     // at least 24 younger vector memory operations (its own V loads and the next pair's DMAs
-    // and V loads), so vmcnt(24) means the pair has landed. The compiler's own waits for the V
-    // registers count only its own loads and so also cover the DMAs issued before them.
+    // and V loads), so vmcnt(24) means the pair has landed; a wavefront's last pair by at least its
+    // own eight V loads. The compiler's own waits for the V registers count only its own loads and
+    // so also cover the DMAs issued before them.
     auto dma_k = [&](const int (&id)[2], half8_t* slot) {
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // the slot's last reads are done
 #pragma unroll
@@ -767,20 +773,25 @@ __device__ __forceinline__ void decode_mfma_body(
       }
     };
     int idn[2] = {0, 0};
-    auto stepk = [&](int p, VRow (&vr)[2][4], half8_t* slot) {
+    auto stepk = [&](int p, VRow (&vr)[2][4], half8_t* slot, auto left) {
+      constexpr int kLeft = decltype(left)::value;
       int idnn[2];
-      ids_of(last_or(p + 3 * NW, last_or(p + 2 * NW, last_or(p + NW, p))), idnn);
+      if constexpr (kLeft == kLoop) ids_of(last_or(p + 3 * NW, p + NW), idnn);
       const int ba = blk_lo + 2 * p;
       const int ta = ba * kBlockSize + 4 * g, tb = ta + kBlockSize;
       half8_t kf[2][KK];
-      asm volatile("s_waitcnt vmcnt(24)" ::: "memory");    // this pair's K has landed
+      // this pair's K has landed
+      if constexpr (kLeft == kLast) {
+        asm volatile("s_waitcnt vmcnt(8)" ::: "memory");
+      } else {
+        asm volatile("s_waitcnt vmcnt(24)" ::: "memory");
+      }
 #pragma unroll
       for (int j = 0; j < 2; ++j)
 #pragma unroll
         for (int kk = 0; kk < KK; ++kk) kf[j][kk] = slot[256 * j + 16 * c + ((4 * kk + g) ^ c)];
-      if (newest(p)) {
-        patch_k(kf);
-        patch_v(vr);
+      if constexpr (kLeft != kLoop) {
+        if (newest(p)) take_new_row(kf, vr);
       }
       float4_t sa = zero4, sb = zero4;
 #pragma unroll
@@ -803,14 +814,18 @@ __device__ __forceinline__ void decode_mfma_body(
           return vt_operand<VW>(vr[0], vr[1], t, tail_a, kMasked, ta, tb, tok_hi);
         });
       };
-      if ((ba + 2) * kBlockSize > tok_hi)
+      if (kLeft != kLoop && (ba + 2) * kBlockSize > tok_hi)
         finish(std::true_type());
       else
         finish(std::false_type());
-      dma_k(idn, slot);
-      load_v(idn, vr);
-      idn[0] = idnn[0];
-      idn[1] = idnn[1];
+      if constexpr (kLeft == kLoop) {
+        __builtin_amdgcn_sched_barrier(0);
+        dma_k(idn, slot);
+        load_v(idn, vr);
+        __builtin_amdgcn_sched_barrier(0);
+        idn[0] = idnn[0];
+        idn[1] = idnn[1];
+      }
     };
     VRow vA[2][4], vB[2][4];
     int p = w;
@@ -831,23 +846,24 @@ __device__ __forceinline__ void decode_mfma_body(
       load_v(id0, vA);
       load_v(id1, vB);
       ids_of(last_or(p + 2 * NW, last_or(p + NW, p)), idn);
-    } else {
-      request_rows();
-      // pending loads of this path would be waited for where the paths join
-      __builtin_amdgcn_s_waitcnt(kWaitVmcntZero);
-    }
-    rotate_and_write();
-    // The loop sits on the prologue's path only, so the compiler's wait state at its head is the
-    // prologue's (q and the prologue loads in flight), not that of a path with no loads.
-    if (p < npairs) {
+      rotate_rows();
+      check_slot();
       if (mapped) poison = poison || stale();
-      for (; p < npairs; p += 2 * NW) {
-        stepk(p, vA, kslot0);
-        if (p + NW >= npairs) break;
-        stepk(p + NW, vB, kslot1);
+      for (; p + 3 * NW < npairs; p += 2 * NW) {
+        stepk(p, vA, kslot0, Left<kLoop>());
+        stepk(p + NW, vB, kslot1, Left<kLoop>());
       }
-    } else if (mapped) {
-      poison = poison || stale();
+      if (p + 2 * NW < npairs) {
+        stepk(p, vA, kslot0, Left<kLoop>());
+        stepk(p + NW, vB, kslot1, Left<kLastButOne>());
+        stepk(p + 2 * NW, vA, kslot0, Left<kLast>());
+      } else {
+        stepk(p, vA, kslot0, Left<kLastButOne>());
+        if (p + NW < npairs) stepk(p + NW, vB, kslot1, Left<kLast>());
+      }
+    } else {
+      check_slot();
+      if (mapped) poison = poison || stale();
     }
     // the ring's memory is reused by the merge below: every DMA of every wavefront has landed
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
@@ -858,15 +874,17 @@ __device__ __forceinline__ void decode_mfma_body(
     int idk[2] = {0, 0}, idv[2] = {0, 0};        // next K refill / next V refill (two pairs on)
     // Pair p: S^T from kf, refill kf with pair p + NW, softmax, P.V from vr, refill vr with pair
     // p + 2 NW.
-    auto step = [&](int p, VRow (&vr)[2][4]) {
+    auto step = [&](int p, VRow (&vr)[2][4], auto left) {
+      constexpr int kLeft = decltype(left)::value;
       int idk_next[2], idv_next[2];
-      ids_of(last_or(p + 2 * NW, last_or(p + NW, p)), idk_next);
-      ids_of(last_or(p + 3 * NW, last_or(p + 2 * NW, last_or(p + NW, p))), idv_next);
+      if constexpr (kLeft == kLoop) {
+        ids_of(last_or(p + 2 * NW, p + NW), idk_next);
+        ids_of(last_or(p + 3 * NW, last_or(p + 2 * NW, p + NW)), idv_next);
+      }
       const int ba = blk_lo + 2 * p;
       const int ta = ba * kBlockSize + 4 * g, tb = ta + kBlockSize;
-      if (newest(p)) {
-        patch_k(kf);
-        patch_v(vr);
+      if constexpr (kLeft != kLoop) {
+        if (newest(p)) take_new_row(kf, vr);
       }
       float4_t sa = zero4, sb = zero4;             // S^T = K . Q^T: two independent MFMA chains
 #pragma unroll
@@ -879,7 +897,7 @@ __device__ __forceinline__ void decode_mfma_body(
           sb = mfma16x16x16(lo4(kf[1][kk]), lo4(qf[kk]), sb);
         }
       }
-      load_k(idk, kf);
+      if constexpr (kLeft != kLast) load_k(idk, kf);
       // Only the last pair of a range can reach past tok_hi (token 0 of block a never does), so
       // the masked form is a separate, rarely taken path and the common one carries no selects.
       auto finish = [&](auto masked) {
@@ -898,15 +916,19 @@ __device__ __forceinline__ void decode_mfma_body(
           return vt_operand<VW>(vr[0], vr[1], t, tail_a, kMasked, ta, tb, tok_hi);
         });
       };
-      if ((ba + 2) * kBlockSize > tok_hi)
+      if (kLeft != kLoop && (ba + 2) * kBlockSize > tok_hi)
         finish(std::true_type());
       else
         finish(std::false_type());
-      load_v(idv, vr);
-      idk[0] = idk_next[0];
-      idk[1] = idk_next[1];
-      idv[0] = idv_next[0];
-      idv[1] = idv_next[1];
+      if constexpr (kLeft == kLoop) {
+        __builtin_amdgcn_sched_barrier(0);
+        load_v(idv, vr);
+        __builtin_amdgcn_sched_barrier(0);
+        idk[0] = idk_next[0];
+        idk[1] = idk_next[1];
+        idv[0] = idv_next[0];
+        idv[1] = idv_next[1];
+      }
     };
     int p = w;
     if (p < npairs) {
@@ -920,23 +942,33 @@ __device__ __forceinline__ void decode_mfma_body(
         ids_of(p, id0);
         ids_of(last_or(p + NW, p), id1);
       }
-      load_k(id0, kf);
       request_rows();
+      load_k(id0, kf);
       load_v(id0, vA);
       load_v(id1, vB);
       ids_of(last_or(p + NW, p), idk);
       ids_of(last_or(p + 2 * NW, last_or(p + NW, p)), idv);
+      rotate_rows();
+      check_slot();
+      if (mapped) poison = poison || stale();
+      // D = 256 has no registers for a form with three pairs left: its loop's last refill may
+      // repeat a pair.
+      constexpr int kThree = D < 256 ? 3 : 2;
+      for (; p + kThree * NW < npairs; p += 2 * NW) {
+        step(p, vA, Left<kLoop>());
+        step(p + NW, vB, Left<kLoop>());
+      }
+      if (kThree == 3 && p + 2 * NW < npairs) {
+        step(p, vA, Left<kLoop>());
+        step(p + NW, vB, Left<kLastButOne>());
+        step(p + 2 * NW, vA, Left<kLast>());
+      } else {
+        step(p, vA, Left<kLastButOne>());
+        if (p + NW < npairs) step(p + NW, vB, Left<kLast>());
+      }
     } else {
-      request_rows();
-      // pending loads of this path would be waited for where the paths join
-      __builtin_amdgcn_s_waitcnt(kWaitVmcntZero);
-    }
-    rotate_and_write();
-    if (mapped) poison = poison || stale();
-    for (; p < npairs; p += 2 * NW) {
-      step(p, vA);
-      if (p + NW >= npairs) break;
-      step(p + NW, vB);
+      check_slot();
+      if (mapped) poison = poison || stale();
     }
   }
   l = rows_sum(l);
