@@ -317,6 +317,12 @@ int ts_w8a16_gemm(const void* x, int64_t ldx, const int8_t* wq, const void* scal
                   void* workspace, size_t workspace_bytes, void* stream);
 
 /*
+ * The block tile that the library's own plan takes for this product (of the gated form N = 2I), for
+ * tests and traces: weight rows << 16 | activation rows << 4 | K groups, 0 where another kernel runs.
+ */
+int32_t ts_w8a16_plan_tile(int32_t M, int32_t N, int32_t K, int32_t cu_count);
+
+/*
  * The same product with a named kernel variant, the choice a tuning table makes for a shape
  * bucket (the role of the reference's per-bucket W8A16 configs, autopilot/tuner.py:116-134 and
  * ops/triton_ops.py:74-86): variant 0 = the library's own plan (as ts_w8a16_gemm), 1 = weight

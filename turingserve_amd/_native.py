@@ -74,6 +74,7 @@ SIGNATURES = {
                                           _i32, _p, _p, _i32, _i32, _i32, _i32, _i32, _i32, _i32,
                                           _i32, _f32, _i32, _i32, _p, _sz, _p]),
     "ts_w8a16_workspace_bytes": (_sz, [_i32, _i32, _i32, _i32]),
+    "ts_w8a16_plan_tile": (_i32, [_i32, _i32, _i32, _i32]),
     "ts_w8a16_gemm": (ctypes.c_int, [_p, _i64, _p, _p, _i32, _p, _p, _i64, _i32, _i32, _i32, _p,
                                      _sz, _p]),
     "ts_w8a16_workspace_bytes_v": (_sz, [_i32, _i32, _i32, _i32, _i32, _i32]),

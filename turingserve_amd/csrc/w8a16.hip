@@ -1371,48 +1371,63 @@ enum GemmTile : int {
   kTileNone = 0, kTile256x256, kTile256x192, kTile128x128k2, kTile128x96k4, kTile128x64k4,
   kTile64x96k4, kTile128x96k2, kTile128x64k2, kTile128x32k4, kTile64x32k4
 };
-struct TileSize { int rows, cols, bk; };
-constexpr TileSize kTileSizes[] = {{0, 0, 0},     {256, 256, 64}, {256, 192, 64},
-                                   {128, 128, 128}, {128, 96, 128}, {128, 64, 128},
-                                   {64, 96, 128}, {128, 96, 64},  {128, 64, 64},
-                                   {128, 32, 128}, {64, 32, 128}};
+struct TileSize { int rows, cols, bk, groups; };
+constexpr TileSize kTileSizes[] = {{0, 0, 0, 0},       {256, 256, 64, 1}, {256, 192, 64, 1},
+                                   {128, 128, 128, 2}, {128, 96, 128, 4}, {128, 64, 128, 4},
+                                   {64, 96, 128, 4},   {128, 96, 64, 2},  {128, 64, 64, 2},
+                                   {128, 32, 128, 4},  {64, 32, 128, 4}};
 static int64_t tile_count(int t, int M, int N) {
   const TileSize& s = kTileSizes[t];
   return (int64_t)((N + s.rows - 1) / s.rows) * ((M + s.cols - 1) / s.cols);
 }
 
-// Which block tile past M = 64, for a product whose wide plan does not split K (cold weights,
-// wide plan -> block tile; one workgroup per CU unless said otherwise):
+// Which block tile past M = 64, for a product whose wide plan (`wide_cols` columns per tile) does not
+// split K (cold weights, wide plan -> block tile; one workgroup per CU unless said otherwise):
 //  * 256 x 256 or 256 x 192 where the output fills its resident rounds well enough that the
-//    larger operand blocks pay: at least 9/10 (16384 x 8192 at M = 2048: 620 -> 482 us) and 25/32
-//    of rounds x CUs x tile (17920 x 1536: M = 560 44.8 -> 41.3 us, M = 1856 138 -> 121 us; at
-//    M = 1024 and 1400, 0.73 and 0.67 of the rounds, they measured 4 and 8 % slower);
+//    larger operand blocks pay, in parts of rounds x CUs x tile: at least 9/10 (16384 x 8192 at
+//    M = 2048: 620 -> 482 us); for 256 x 192 25/32 of a single round (17920 x 1536 at M = 560 44.8 ->
+//    41.3 us, 9728 x 896 at M = 1024 31.7 -> 28.9) and 13/16 of several (17920 x 1536 at M = 1152, 0.82:
+//    83.1 -> 81.1, M = 1856, 0.88: 138 -> 121; at 0.79 17920 x 1536 at M = 1664 is level and 9728 x 896
+//    at M = 2048 went 53.4 -> 54.7);
 //  * the smallest of 64 x 96, 128 x 64, 128 x 96 (four K groups) and 128 x 128 (two) that fits one
 //    round of one workgroup per CU, so that the most CUs share the work, while it covers 0.7
 //    of them (2048 x 1536: M = 560 / 768 / 1400 / 1856 11.5 / 11.9 / 17.8 / 20.7 -> 10.3 / 10.6 /
 //    16.0 / 18.5 us; 1536 x 1536 at M = 1856 20.0 -> 16.2; 1536 x 8960: M = 1400 / 1856 71.1 / 85.8 ->
-//    55.9 / 60.0; below the 0.7, 128 x 32 wide tiles stay: 1536 x 1536 at M = 560 8.9 against 9.9);
+//    55.9 / 60.0; below the 0.7, 128 x 32 wide tiles stay: 1536 x 1536 at M = 560 8.9 against 9.9).
+//    Four 128 x 32 wide tiles per CU stay too (1152 x 896 at M = 896 6.7 against 7.6; 2048 x 1536 at
+//    M = 512 with RoPE and the cache write, whose tiles hold whole heads, 11.1 against 12.6), and 128 x 64
+//    wide tiles at short K, where the four groups' meeting is not made up for (9728 x 896, gated:
+//    M = 160 / 192 10.1 / 10.2 against 10.4 / 10.6; 1152 x 896 at M = 1664 9.0 against 9.2; from K = 1536
+//    on the block tile is 2 to 12 % faster);
 //  * 128 x 96 or 128 x 64 with two K groups and two workgroups per CU, whichever pads fewer rows,
-//    for a wide product of few rows (17920 x 1536: M = 72 / 130 / 192 / 256 20.8 / 23.7 / 25.1 /
-//    31.0 -> 17.4 / 22.2 / 24.1 / 29.2 us).
-static int pick_tile(int M, int N, int K, int cus) {
+//    for a wide product of few rows (17920 x 1536: M = 72 / 130 / 192 / 256 19.5 / 23.7 / 25.1 /
+//    31.0 -> 16.9 / 22.2 / 24.1 / 29.2 us). Where 128 x 128 wide tiles fit one round of one workgroup per
+//    CU, only 128 x 96 (M = 97 to 128 took 128 x 64 tiles from 7 % faster to 5 % slower: 17920 x 512 11.8 ->
+//    10.9, 17920 x 3072 31.6 -> 33.5, 9728 x 896 10.0 -> 10.5).
+constexpr int kTile128x64k4MinK = 1536;
+static int pick_tile(int M, int N, int K, int cus, int wide_cols) {
   if (K % kTileBK != 0) return kTileNone;
+  auto rounds = [&](int t) { return (tile_count(t, M, N) + cus - 1) / cus; };
   auto fills = [&](int t, int num, int den) {
-    const int64_t rounds = (tile_count(t, M, N) + cus - 1) / cus;
     return (int64_t)M * N * den >=
-           num * rounds * cus * ((int64_t)kTileSizes[t].rows * kTileSizes[t].cols);
+           num * rounds(t) * cus * ((int64_t)kTileSizes[t].rows * kTileSizes[t].cols);
   };
   if (fills(kTile256x256, 9, 10)) return kTile256x256;
-  if (fills(kTile256x192, 25, 32)) return kTile256x192;
-  if (K % 128 == 0 && tile_count(kTile128x128k2, M, N) <= cus) {
-    for (int t : {kTile64x96k4, kTile128x64k4, kTile128x96k4, kTile128x128k2})
-      if (tile_count(t, M, N) <= cus) return tile_count(t, M, N) * 10 >= 7LL * cus ? t : kTileNone;
+  if (rounds(kTile256x192) == 1 ? fills(kTile256x192, 25, 32) : fills(kTile256x192, 13, 16))
+    return kTile256x192;
+  const bool one_round = tile_count(kTile128x128k2, M, N) <= cus;
+  if (K % 128 == 0 && one_round) {
+    for (int t : {kTile64x96k4, kTile128x64k4, kTile128x96k4, kTile128x128k2}) {
+      if (tile_count(t, M, N) > cus) continue;
+      if (tile_count(t, M, N) * 10 < 7LL * cus) break;   // and a larger one covers fewer CUs
+      return wide_cols == 32 || (t == kTile128x64k4 && K < kTile128x64k4MinK) ? kTileNone : t;
+    }
   }
   if (M <= 256 && tile_count(kTile128x96k2, M, N) * 2 > cus) {
     const int r64 = (M + 63) / 64 * 64, r96 = (M + 95) / 96 * 96;
     const int t = r64 <= r96 && tile_count(kTile128x64k2, M, N) <= 2LL * cus ? kTile128x64k2
                                                                             : kTile128x96k2;
-    if (tile_count(t, M, N) <= 2LL * cus) return t;
+    if (tile_count(t, M, N) <= 2LL * cus && !(one_round && t == kTile128x64k2)) return t;
   }
   return kTileNone;
 }
@@ -1558,7 +1573,7 @@ static GemmPlan plan_gemm_v(int M, int N, int K, int cus, int variant, int split
   GemmPlan p = plan_gemm_wide(M, N, K, cus, variant, splits, glu);
   if (variant != kVarAuto || p.gv > 0) return p;
   if (M > 64) {
-    if (p.splits == 1) p.tile = pick_tile(M, N, K, cus);
+    if (p.splits == 1) p.tile = pick_tile(M, N, K, cus, p.bm);
     return p;
   }
   const int t = pick_small_tile(M, N, K, cus, p.splits);
@@ -1584,6 +1599,12 @@ using namespace ts;
 extern "C" size_t ts_w8a16_workspace_bytes(int32_t M, int32_t N, int32_t K, int32_t cu_count) {
   if (M <= 0 || N <= 0 || K <= 0) return 0;
   return gemm_workspace(plan_gemm(M, N, K, cu_count > 0 ? cu_count : 256), M, N);
+}
+
+extern "C" int32_t ts_w8a16_plan_tile(int32_t M, int32_t N, int32_t K, int32_t cu_count) {
+  if (M <= 0 || N <= 0 || K <= 0) return 0;
+  const TileSize& t = kTileSizes[plan_gemm(M, N, K, cu_count > 0 ? cu_count : 256).tile];
+  return t.rows << 16 | t.cols << 4 | t.groups;
 }
 
 static bool variant_valid(int variant, int splits, int M) {
@@ -1652,7 +1673,8 @@ static int w8a16_launch(const half_t* xp, int64_t ldx, const int8_t* wq, const v
   case ID: {                                                                                       \
     using Shape = TileShape<__VA_ARGS__>;                                                          \
     static_assert(Shape::kTN == kTileSizes[ID].rows && Shape::kTM == kTileSizes[ID].cols &&        \
-                  Shape::kBK == kTileSizes[ID].bk, "the planner's table");                         \
+                  Shape::kBK == kTileSizes[ID].bk && Shape::kGroups == kTileSizes[ID].groups,      \
+                  "the planner's table");                                                          \
     w8a16_tile_kernel<__VA_ARGS__><<<grid, Shape::kThreads, 0, s>>>(                               \
         xp, ldx, wq, scale, scale_is_fp16, bp, yp, ldy, M, N, K, io);                              \
     break;                                                                                         \

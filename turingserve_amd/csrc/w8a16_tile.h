@@ -24,7 +24,7 @@ namespace ts {
 // that barrier, which every wavefront passes with its reads of the stage complete (lgkmcnt 0).
 template <int IN, int JM, int WN, int WM, int KG, int SUB, int S>
 struct TileShape {
-  static constexpr int kThreads = 64 * WN * WM * KG;
+  static constexpr int kThreads = 64 * WN * WM * KG, kGroups = KG;
   static constexpr int kTN = 32 * IN * WN, kTM = 32 * JM * WM, kBK = 64 * SUB;
   static constexpr int kWBytes = kTN * kBK, kXBytes = kTM * kBK * 2;
   static constexpr int kStage = kWBytes + kXBytes;
