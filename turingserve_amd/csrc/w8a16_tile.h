@@ -62,7 +62,7 @@ __global__ void __launch_bounds__(64 * WN * WM * KG) w8a16_tile_kernel(
   constexpr int QW = 4 * SUB / KG;                        // K slices per wavefront and step
   static_assert(XD * NT == TM * 8 * SUB && WD * NT == TN * 4 * SUB, "tiles split over the threads");
   static_assert(QW == 2 || QW == 4, "a group's slices stay inside one 64-column sub-step");
-  static_assert((S - 2) * BATCH < 64, "vmcnt holds 6 bits");
+  static_assert((S - 1) * BATCH < 64, "vmcnt holds 6 bits; the first wait leaves S - 1 batches");
   static_assert(S >= 2 && T::kLds + 8 * TN <= 160 * 1024, "LDS of one CU");
   __shared__ __align__(16) char smem[T::kLds];
   __shared__ float s_sc[TN], s_bs[TN];
