@@ -1640,8 +1640,10 @@ static int w8a16_launch(const half_t* xp, int64_t ldx, const int8_t* wq, const v
     p = plan_gemm_v(M, N, K, cus, kVarSkinny, 0, glu);   // the VALU path's alignment not met
   if (p.tile != kTileNone && !aligned(wq, 16)) {  // the block tiles' weight DMA
     p = plan_gemm_wide(M, N, K, cus, kVarAuto, 0, glu);
-    if (p.splits > 1)                             // the plan's size named no workspace
-      p = plan_gemm_wide(M, N, K, cus, kVarSkinny, 0, glu);
+    // The plan's size named no workspace; without the weight DMA the skinny kernel is the faster one
+    // all the same (8-byte aligned weights, M = 33 / 64: 2048 x 1536 11.2 / 11.5 us split over K, 9.1 /
+    // 11.2 skinny, 1152 x 896 10.2 / 10.2 and 6.6 / 8.0).
+    if (p.splits > 1) p = plan_gemm_wide(M, N, K, cus, kVarSkinny, 0, glu);
   }
   if (glu && p.bm == 32) p.bm = 64;               // GLU tiles pair 32-row subtiles (same splits)
   const size_t need = gemm_workspace(p, M, N);
