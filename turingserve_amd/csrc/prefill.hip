@@ -16,7 +16,11 @@ namespace {
 //    launch and first-load latency and no split pays: 2 rows on 0 4.1 / 4.7 / 5.8, 256 on 0 7.6 / 8.7
 //    / 7.2, 512 on 0 9.7 / 12.6 / 9.8, 300 on 700 13.3 and 15.0 with two groups, 512 on 1000 17.6 and
 //    17.9 (past one per CU: six chunks of 300 on 0 14.5 / 9.6 / 9.5); a batch of a few tiles, whose
-//    keys split well, leaves it at 640 keys (30 rows on 700 11.1 and 10.1, 16 on 500 9.2 and 9.9);
+//    keys split well, leaves it at 640 keys (30 rows on 700 11.1 and 10.1, 16 on 500 9.2 and 9.9), a
+//    single chunk whose 64-row tiles give most CUs work, which a split can only double, later than
+//    others (two layers, stream and split tiles: 700 on 900 on 8 heads 42.1 / 43.8, 1024 on 596 42.0 /
+//    44.9, on 736 44.1 / 45.8 and on 926 47.5 / 46.6, 500 on 1080 on 14 heads 39.2 / 40.2; three of 240
+//    on 1340 on 8 heads 44.9 / 39.2);
 //  * two key groups halve a workgroup's chain of key steps and give a short batch twice the
 //    workgroups: 1024 on 0 19.3 / 18.2 / 15.2, 2048 on 0 43.8 / 32.2 / 30.0, 2000-token prefix with
 //    16 rows 19.5 / 11.5 / 11.0, five ragged chunks 35.7 / 31.8 / 23.8;
@@ -34,6 +38,7 @@ struct Plan64 {
   TilePlan tile;
 };
 constexpr int kStream64Keys = 1536, kStream64KeysFew = 640;
+constexpr int kStream64KeysThird = 1664, kStream64KeysMost = 1760;   // a single chunk
 constexpr int kLong64Steps = 64, kFew64 = 8, kSplit64Steps = 16, kSplit64From = 28;
 
 TilePlan tile_plan64(int ks, int min_steps, int P, int H, int max_query_len, int max_seq_len,
@@ -51,13 +56,15 @@ Plan64 plan64(int P, int H, int64_t num_tokens, int max_query_len, int max_seq_l
     const int64_t a = (int64_t)cdiv(max_query_len, rows) * P, b = num_tokens / rows + P;
     return (a < b ? a : b) * H;
   };
-  const bool few = tiles(tile_rows(2)) * kFew64 <= cus;
-  if (tiles(kPsRows) <= cus && seq <= (few ? kStream64KeysFew : kStream64Keys))
-    return {kStream64, {}};
+  const int64_t t2 = tiles(tile_rows(2));
+  const bool few = t2 * kFew64 <= cus;
+  int stream_keys = few ? kStream64KeysFew : kStream64Keys;
+  if (P == 1 && t2 * 3 > cus) stream_keys = t2 * 16 >= 7LL * cus ? kStream64KeysMost : kStream64KeysThird;
+  if (tiles(kPsRows) <= cus && seq <= stream_keys) return {kStream64, {}};
   const int ks = cdiv(seq, kTileKeys) >= kLong64Steps || tiles(kTileRows) * 4 > 7LL * cus ? 1 : 2;
   const int min_steps = ks == 1 || few ? kPrefillMinSteps : kSplit64Steps;
   const bool pays =
-      ks == 1 || tiles(tile_rows(2)) * 2 <= cus || cdiv(seq, kTileKeys) >= kSplit64From;
+      ks == 1 || t2 * 2 <= cus || cdiv(seq, kTileKeys) >= kSplit64From;
   return {ks, tile_plan64(ks, min_steps, P, H, max_query_len, max_seq_len, cus, split && pays)};
 }
 
