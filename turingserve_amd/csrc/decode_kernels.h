@@ -1168,7 +1168,7 @@ static_assert(2 * kDecodeWaves == kMapPairs, "split map entries hold two pairs p
 
 // Workgroups of decode_mfma_kernel resident per CU (4 wavefronts each, one per SIMD), from the
 // kernel's VGPR use (512 per SIMD lane): 6 waves per SIMD up to D = 32, 3 at D = 64, 2 at
-// D = 128 (236 VGPRs), 1 at D = 256.
+// D = 128 (203 to 256 VGPRs), 1 at D = 256.
 static int decode_wgs_per_cu(int D) { return D <= 32 ? 6 : (D == 64 ? 3 : (D == 128 ? 2 : 1)); }
 
 struct SplitPlan {

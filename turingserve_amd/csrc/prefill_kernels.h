@@ -219,10 +219,11 @@ __global__ void __launch_bounds__(NW * 64) prefill_stream_kernel(
 // in LDS at the end: a workgroup alone on its CU is bound by the chain of one step (reads, MFMAs,
 // softmax, ~1.2 us at D = 64), which two groups halve (five ragged chunks, 2060 rows on 14 heads:
 // 31.8 -> 23.8 us; the 32-row stream kernel 35.7). Every 64-key
-// step (four 16-token blocks) is staged once in LDS and shared by the four wavefronts: K in its
-// natural [key][dim] layout, V transposed to [dim][key] (16 bytes of padding per row keep the
-// 16-lane groups of each 16-byte read on distinct banks). Wavefront w stages block w of the
-// step, so its block-table entry is one scalar load. Per wavefront and step (lane l = 32 h + r):
+// step (four 16-token blocks) is staged once in LDS and shared by the wavefronts of its key group: K
+// in its natural [key][dim] layout, V transposed to [dim][key] (16 bytes of padding per row keep the
+// 16-lane groups of each 16-byte read on distinct banks). Wavefront w of one group of four stages
+// block w of the step, wavefront rw of two groups of two the blocks rw and rw + 2 of its group's
+// step, each block-table entry a scalar load. Per wavefront and step (lane l = 32 h + r):
 //   S^T[32 keys][32 rows] = K . Q^T    v_mfma_f32_32x32x16_f16, two key halves x D/16 k-steps;
 //       lane (r, h) of the result holds keys 8j + 4h + i (j, i = 0..3) of query row r, so every
 //       per-row softmax statistic sits in lanes r and r + 32;
@@ -374,8 +375,8 @@ __device__ __forceinline__ PrefillSeq prefill_seq(const int* __restrict__ qsl,
   return p;
 }
 
-// Workspace of the split path: per-split rows O (unnormalised) [slots_total][128][D] fp32, then
-// (m, l) pairs [slots_total][128][2] fp32, slots_total = P * H * slots.
+// Workspace of the split path: per-split rows O (unnormalised) [slots_total][tile_rows(KS)][D] fp32,
+// then (m, l) pairs [slots_total][tile_rows(KS)][2] fp32, slots_total = P * H * slots.
 template <int D, int KS>
 __device__ __forceinline__ void prefill_tile_body(
     const half_t* __restrict__ q, int64_t q_st, int64_t q_sh, half_t* __restrict__ out,
