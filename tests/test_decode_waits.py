@@ -66,6 +66,17 @@ def test_two_pairs_stay_in_flight(assembly, src, name):
     events += sum((ev for _, ev in blocks[ask + 1:mfma]), [])
     assert "bar" not in events
     assert all(e >= 16 for e in events if isinstance(e, int)), events
+    # the written-out waits for the K ring count on this order: two pairs' K by DMA, then (the tables,
+    # the new row and) both pairs' V; at each refill a pair's K by eight DMAs, then its V
+    order = [e for _, ev in blocks[:mfma] for e in ev if e in ("dma", "load")]
+    if "dma" in order:
+        first = order.index("dma")
+        assert order[first:first + 16] == ["dma"] * 16 and order.count("dma") == 16
+        assert order[first + 16:].count("load") >= 16
+        for _, ev in blocks[mfma:]:
+            refill = [e for e in ev if e in ("dma", "load")]
+            if "dma" in refill:
+                assert refill == (["dma"] * 8 + ["load"] * 8) * (len(refill) // 16)
     loops = [ev for loop, ev in blocks if loop and "mfma" in ev]
     assert loops
     for ev in loops:
